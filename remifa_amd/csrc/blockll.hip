@@ -18,8 +18,8 @@
 // order). That is the
 // reference's per-ib-block GEMM (one update over every column of the outer
 // block left of the ib block) followed by its panel kernel
-// (src/lu_nopiv.cu:123-170, 251-326); the slice kernels (subpanel.hip)
-// split the same update sum at the slice boundary instead.
+// (src/lu_nopiv.cu:123-170, 251-326); the slice kernel (slice.hpp)
+// splits the same update sum at the slice boundary instead.
 //
 // Two launches per outer block, on the handle's stream:
 //  * the diagonal kernel, one workgroup: for each slice, the tile's update
@@ -572,7 +572,7 @@ __device__ void diagonal_role(const BlkArgs& g, DiagLds& S) {
     for (int jj = 0; jj < TP; ++jj) x[jj] = S.f.tt[i][cb + jj];
     __syncthreads();
     // 2. the factorization (ib = 32)
-    tile_factor<MODE, false, 32>(S.f.fac, x, 32, w, i);
+    tile_factor<MODE, 32>(S.f.fac, x, 32, w, i);
     __syncthreads();
     const float rk = S.f.fac.R[i];
     // 3. the factored tile: fp16 factors, the slice table (LDS, then copied

@@ -267,6 +267,18 @@ int fp8_gemm_launch(remifa_handle_t h, int out_t, int64_t m, int64_t n, int64_t 
                     void* c, int64_t ldc, const void* cin = nullptr, int cin_t = 0,
                     int64_t ldcin = 0);
 
+// the diagonal tile that the last slice of an inner factorization left in a
+// slot of the workspace (slice.hip): its place in the matrix (and in the
+// fp16 mirror), copied there by the next slice's launch or the final one
+struct SlicePending {
+  float* slots = nullptr;  // two slots, taken in turn
+  int next = 0;            // slices so far
+  int sw = 0;              // width of the pending tile (0: none)
+  void* a = nullptr;
+  half_t* cp = nullptr;
+  int64_t first_col = -1;  // column of the first slice
+};
+
 int copy2d_launch(remifa_handle_t h, size_t elt, int64_t m, int64_t n, const void* a, int64_t lda,
                   void* b, int64_t ldb);
 

@@ -8,11 +8,12 @@
 // factorization of the block with its ib-granular semantics.
 //
 // The inner factorization runs over slices of pw <= 64 columns (pw a multiple
-// of ib, default 64): each slice is one fused kernel (subpanel.hip) that does
-// the reference's ib loop inside, and the updates between slices are matrix-
-// core GEMMs (LL: the slice's columns/rows minus everything left of it, K =
-// slice offset; RL: a rank-pw update after it). pw = ib reproduces the
-// reference's structure of one panel per ib columns.
+// of ib, default 64): each slice is one launch (slice.hip) that subtracts the
+// earlier slices of the outer block (LL: one sum; RL: slice by slice, as the
+// rank-pw updates after each slice would) and does the reference's ib loop.
+// fp16-accumulated sums, and bf16 ones of fp32 buffers, come from update
+// GEMMs between the slices instead. pw = ib reproduces the reference's
+// structure of one panel per ib columns.
 //
 // Differences from the reference, all deliberate:
 //  * no allocation inside the loop: one workspace arena per call (slice
@@ -28,9 +29,15 @@
 
 namespace remifa {
 
-int subpanel_launch(remifa_handle_t h, int T, int I, bool rl, int ib, int64_t cm, int sw, void* l,
-                    int64_t ldl, void* u, int64_t ldu, half_t* cp, int64_t ldcp, float* tab);
-size_t subpanel_table_bytes();
+int slice_launch(remifa_handle_t h, int T, int W, int I, bool rl, int ib, int pw, int64_t m,
+                 int64_t nb, int64_t so, int sw, bool last, void* l, int64_t ldl, void* u,
+                 int64_t ldu, bool store_x, half_t* cp, int64_t ldcp, void* ops, void* a,
+                 int64_t lda, half_t* acp, int64_t ldacp, int64_t col, SlicePending& pend);
+int slice_finish_launch(remifa_handle_t h, int W, int64_t n, const void* d_a, int64_t lda,
+                        int64_t ldacp, const SlicePending& pend, int* info);
+size_t slice_slot_bytes();
+size_t slice_op_bytes(int T, int I, int64_t m, int64_t nb);
+bool slice_updates(int T, int I);
 size_t blockll_workspace_bytes(int64_t m, int64_t nb);
 int* blockll_sync_words(void* base, int64_t m, int64_t nb);
 int blockll_cus(remifa_handle_t h, int64_t updm, int64_t in);
@@ -40,20 +47,6 @@ int blockll_launch(remifa_handle_t h, void* base, int64_t m, int64_t nb, int64_t
                    half_t* a, int64_t lda, int* seq);
 
 namespace {
-
-__global__ void info_kernel(int64_t n, const void* a, int64_t lda, int t, int* info) {
-  // one workgroup: first column k with u_kk == 0 or not finite (1-based)
-  __shared__ int first;
-  if (threadIdx.x == 0) first = 0x7fffffff;
-  __syncthreads();
-  for (int64_t k = threadIdx.x; k < n; k += blockDim.x) {
-    float v = (t == REMIFA_R_16F) ? (float)((const half_t*)a)[k + k * lda]
-                                  : ((const float*)a)[k + k * lda];
-    if (v == 0.0f || !__builtin_isfinite(v)) atomicMin(&first, (int)(k + 1));
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) *info = first == 0x7fffffff ? 0 : first;
-}
 
 __global__ void zero_int_kernel(int* p, int n) {
   int i = blockIdx.x * 256 + threadIdx.x;
@@ -82,12 +75,22 @@ size_t gemm_reserve(int64_t m, int64_t nb) {
   return std::min<size_t>((size_t)256 << 20, std::max<size_t>((size_t)16 << 20, full));
 }
 
+// the handle stream's part of the arena past the fixed areas: the split-K
+// partials of its update GEMMs and, while it runs the slices of an outer
+// block (no split-K update runs on that stream then), the slices' operand
+// copies
+size_t main_reserve(const remifa_lu_config_t& c, int T, int64_t m, int64_t nb) {
+  const size_t op = slice_updates(T, c.I) ? slice_op_bytes(T, c.I, m, nb) : 0;
+  return std::max(gemm_reserve(m, nb), op);
+}
+
 struct Ctx {
   remifa_handle_t h;
   remifa_lu_config_t c;
   int64_t ib;
-  int pw;      // slice width of the inner factorization
-  float* tab;  // the slice's published diagonal tile
+  int pw;             // slice width of the inner factorization
+  void* ops;          // the slices' operand copies
+  SlicePending pend;  // the last slice's tile
 };
 
 int gemm(Ctx& x, int ctype, int out_t, int64_t m, int64_t n, int64_t k, const void* a,
@@ -102,41 +105,61 @@ inline void* at(void* p, int t, int64_t i, int64_t j, int64_t ld) {
   return (char*)p + (i + j * ld) * (int64_t)dtype_size(t);
 }
 
-// Inner left-looking factorization of one outer block: m x n block column
-// `l` and n x m block row `u` (columns n.. beyond the diagonal block), both
-// in precision T (l == u when factoring in place). cpy/ldcp: fp16 mirror of
-// this block's factors; when T = fp32 and the inner update is a TC type its
-// operands are read from the mirror (the reference's d_a_cpy,
-// src/lu_nopiv_inner_ll.hxx:225-265). `mirror`: write the factors to cpy.
-int inner_ll(Ctx& x, int T, int64_t m, int64_t n, void* l, int64_t ldl, void* u, int64_t ldu,
-             void* cpy, int64_t ldcp, bool mirror) {
-  const int I = x.c.I;
-  const bool tc_from_copy = (T == REMIFA_R_32F) && I != REMIFA_FP32;
-  if (tc_from_copy) mirror = true;
+// Inner factorization of one outer block: m x n block column `l` and n x m
+// block row `u` (columns n.. beyond the diagonal block), both in precision T
+// (l == u when factoring in place). cpy/ldcp: fp16 mirror of this block's
+// factors, or null (the reference's d_a_cpy,
+// src/lu_nopiv_inner_ll.hxx:225-265). a: the block in the matrix (== l in
+// place), column col of it; store_x: the factors are wanted in l / u and not
+// only in the mirror.
+int inner(Ctx& x, bool rl, int T, int64_t m, int64_t n, int64_t nb, void* l, int64_t ldl, void* u,
+          int64_t ldu, void* cpy, int64_t ldcp, bool store_x, void* a, int64_t lda, int64_t col) {
+  const int I = x.c.I, W = x.c.W;
+  // update GEMMs between the slices where the slice kernel has no sums for
+  // the type; with T = fp32 and an inner TC type their operands are read
+  // from the mirror
+  const bool ext = !slice_updates(T, I);
+  const bool from_copy = (T == REMIFA_R_32F) && I != REMIFA_FP32;
+  const int64_t ldo_l = from_copy ? ldcp : ldl, ldo_u = from_copy ? ldcp : ldu;
+  auto lop = [&](int64_t i, int64_t j) {
+    return (const void*)(from_copy ? at(cpy, REMIFA_R_16F, i, j, ldcp) : at(l, T, i, j, ldl));
+  };
+  auto uop = [&](int64_t i, int64_t j) {
+    return (const void*)(from_copy ? at(cpy, REMIFA_R_16F, i, j, ldcp) : at(u, T, i, j, ldu));
+  };
   for (int64_t so = 0; so < n; so += x.pw) {
     const int sw = (int)std::min<int64_t>(x.pw, n - so);
     const int64_t cm = m - so;
-    if (so > 0) {
-      const void* la = tc_from_copy ? at(cpy, REMIFA_R_16F, so, 0, ldcp) : at(l, T, so, 0, ldl);
-      const int64_t lla = tc_from_copy ? ldcp : ldl;
-      const void* ub = tc_from_copy ? at(cpy, REMIFA_R_16F, 0, so, ldcp) : at(u, T, 0, so, ldu);
-      const int64_t lub = tc_from_copy ? ldcp : ldu;
-      // columns of the slice (:223-246) and its rows right of the diagonal
-      // tile (:249-301): one launch when both take the narrow tiles
-      if (cm > sw) {
-        const void* ub2 = tc_from_copy ? at(cpy, REMIFA_R_16F, 0, so + sw, ldcp)
-                                       : at(u, T, 0, so + sw, ldu);
-        RF_CHECK(gemm_pair_launch(x.h, I, operand_type(I), T, cm, sw, so, la, lla, ub, lub,
-                                  at(l, T, so, so, ldl), ldl, sw, cm - sw, la, lla, ub2, lub,
+    if (ext && !rl && so > 0) {
+      // columns of the slice (src/lu_nopiv_inner_ll.hxx:223-246) and its
+      // rows right of the diagonal tile (:249-301): one launch when both
+      // take the narrow tiles
+      if (cm > sw)
+        RF_CHECK(gemm_pair_launch(x.h, I, operand_type(I), T, cm, sw, so, lop(so, 0), ldo_l,
+                                  uop(0, so), ldo_u, at(l, T, so, so, ldl), ldl, sw, cm - sw,
+                                  lop(so, 0), ldo_l, uop(0, so + sw), ldo_u,
                                   at(u, T, so, so + sw, ldu), ldu));
-      } else {
-        RF_CHECK(gemm(x, I, T, cm, sw, so, la, lla, ub, lub, at(l, T, so, so, ldl), ldl));
-      }
+      else
+        RF_CHECK(gemm(x, I, T, cm, sw, so, lop(so, 0), ldo_l, uop(0, so), ldo_u,
+                      at(l, T, so, so, ldl), ldl));
     }
-    RF_CHECK(subpanel_launch(x.h, T, I, false, (int)x.ib, cm, sw, at(l, T, so, so, ldl), ldl,
-                             at(u, T, so, so, ldu), ldu,
-                             mirror ? (half_t*)at(cpy, REMIFA_R_16F, so, so, ldcp) : nullptr, ldcp,
-                             x.tab));
+    half_t* const cps = cpy ? (half_t*)at(cpy, REMIFA_R_16F, so, so, ldcp) : nullptr;
+    void* const as = at(a, W, so, so, lda);
+    RF_CHECK(slice_launch(x.h, T, W, I, rl, (int)x.ib, x.pw, m, nb, so, sw, so + sw >= n,
+                          at(l, T, so, so, ldl), ldl, at(u, T, so, so, ldu), ldu, store_x, cps,
+                          ldcp, x.ops, as, lda, (void*)cps == as ? nullptr : cps, ldcp, col + so,
+                          x.pend));
+    const int64_t tso = so + sw;
+    if (ext && rl && n > tso) {
+      // rank-sw update of the outer block column
+      // (src/lu_nopiv_inner_rl.hxx:139-163) and of the outer block row beyond
+      // the outer block (:167-193)
+      RF_CHECK(gemm(x, I, T, m - tso, n - tso, sw, lop(tso, so), ldo_l, uop(so, tso), ldo_u,
+                    at(l, T, tso, tso, ldl), ldl));
+      if (m > n)
+        RF_CHECK(gemm(x, I, T, n - tso, m - n, sw, lop(tso, so), ldo_l, uop(so, n), ldo_u,
+                      at(u, T, tso, n, ldu), ldu));
+    }
   }
   return 0;
 }
@@ -246,9 +269,14 @@ int side_stream(remifa_handle_t h) {
   return 0;
 }
 
+// fp16 storage factored in fp32 buffers of one block column and block row
+bool buffered_layout(int algo, const remifa_lu_config_t& c) {
+  return algo == REMIFA_LL && c.W == REMIFA_R_16F && c.IP == REMIFA_R_32F;
+}
+
 size_t lu_workspace_bytes(int algo, const remifa_lu_config_t& c, int64_t m, int64_t n, int64_t nb,
                           bool have_cpy) {
-  size_t b = (subpanel_table_bytes() + 255) & ~(size_t)255;  // slice table
+  size_t b = (2 * slice_slot_bytes() + 255) & ~(size_t)255;  // the slices' tile slots
   if (algo == REMIFA_LL && c.O == REMIFA_BF16_TC32 && c.W == REMIFA_R_16F &&
       c.IP == REMIFA_R_32F)
     b += ((size_t)m * n * 2 + 255) & ~(size_t)255;  // bf16 mirror of the factors
@@ -273,7 +301,8 @@ size_t lu_workspace_bytes(int algo, const remifa_lu_config_t& c, int64_t m, int6
     b += ((size_t)nb * m * 4 + 255) & ~(size_t)255;
     b += gemm_reserve(m, nb);
   }
-  return b + gemm_reserve(m, nb);
+  const int T = buffered_layout(algo, c) ? REMIFA_R_32F : c.W;
+  return b + main_reserve(c, T, m, nb);
 }
 
 int lu_nopiv_impl(remifa_handle_t h, int algo, const remifa_lu_config_t* cfg, int64_t m, int64_t n,
@@ -304,15 +333,15 @@ int lu_nopiv_impl(remifa_handle_t h, int algo, const remifa_lu_config_t* cfg, in
   // slice width: a multiple of ib, at most 64 (handle knob, default 64)
   int pw = h->panel_width > 0 ? h->panel_width : 64;
   pw = std::max<int>((int)c.ib, std::min(64, pw / (int)c.ib * (int)c.ib));
-  Ctx x{h, c, c.ib, pw, nullptr};
-  x.tab = (float*)ar.take(subpanel_table_bytes());
+  Ctx x{h, c, c.ib, pw, nullptr, {}};
+  x.pend.slots = (float*)ar.take(2 * slice_slot_bytes());
   void* cpy = d_cpy;
   int64_t ldc = ldcpy;
   if (need_cpy && !cpy) {
     cpy = ar.take((size_t)m * n * 2);
     ldc = m;
   }
-  const bool buffered = algo == REMIFA_LL && W == REMIFA_R_16F && c.IP == REMIFA_R_32F;
+  const bool buffered = buffered_layout(algo, c);
   void *pl = nullptr, *pu = nullptr;
   int64_t ldpl = m, ldpu = nb;
   if (buffered) {
@@ -355,10 +384,13 @@ int lu_nopiv_impl(remifa_handle_t h, int algo, const remifa_lu_config_t* cfg, in
     f8.su = (uint8_t*)ar.take((size_t)n * f8.lds8);
   }
   h->ws_used = ar.off;
-  // split-K regions: [ar.off, +R) for the handle's stream, [ar.off + R,
-  // +R) for the side stream (the arena's end is lowered while they run)
+  x.ops = (char*)h->ws + ar.off;
+  // split-K regions: [ar.off, +R) for the handle's stream (shared with the
+  // slices' operand copies), [ar.off + R, +R) for the side stream (the
+  // arena's end is lowered while they run)
   const size_t ws_bytes0 = h->ws_bytes;
-  const size_t side_lo = ar.off + gemm_reserve(m, nb), side_hi = side_lo + gemm_reserve(m, nb);
+  const size_t side_lo = ar.off + main_reserve(c, buffered ? REMIFA_R_32F : W, m, nb);
+  const size_t side_hi = side_lo + gemm_reserve(m, nb);
   if (la_layout || la_inplace) h->ws_bytes = side_lo;
   const int64_t nc = (n - 1) / nb + 1;
   // outer update from the mirrors: C[rows r0.., cols c0..] (M x N) -= L[r0.., 0:K] U[0:K, c0..]
@@ -508,7 +540,8 @@ int lu_nopiv_impl(remifa_handle_t h, int algo, const remifa_lu_config_t* cfg, in
           // inner factorization in place; with an fp16 copy (W = fp32 and a
           // TC update) the slice kernels keep it current (:554-563)
           void* cblk = need_cpy ? at(cpy, REMIFA_R_16F, ofs, ofs, ldc) : nullptr;
-          RF_CHECK(inner_ll(x, W, updm, in, blk, ldda, blk, ldda, cblk, ldc, need_cpy));
+          RF_CHECK(inner(x, false, W, updm, in, nb, blk, ldda, blk, ldda, cblk, ldc, true, blk,
+                         ldda, ofs));
           if (fp8) RF_CHECK(mirror8(ofs, in));
         } else {
           // fp16 storage, fp32 inner buffers: pl = block column (updm x in),
@@ -575,7 +608,8 @@ int lu_nopiv_impl(remifa_handle_t h, int algo, const remifa_lu_config_t* cfg, in
             RF_CHECK(blockll_launch(h, blkws, m, nb, updm, in, (const float*)cpl, ldpl,
                                     (const float*)cpu, ldpu, (half_t*)blk, ldda, blk_seq));
           else
-            RF_CHECK(inner_ll(x, REMIFA_R_32F, updm, in, cpl, ldpl, cpu, ldpu, blk, ldda, true));
+            RF_CHECK(inner(x, false, REMIFA_R_32F, updm, in, nb, cpl, ldpl, cpu, ldpu, blk, ldda,
+                           false, blk, ldda, ofs));
           if (fp8) RF_CHECK(mirror8(ofs, in));
           if (bf16m) {
             // round the finished block column (below the diagonal block) and
@@ -599,32 +633,9 @@ int lu_nopiv_impl(remifa_handle_t h, int algo, const remifa_lu_config_t* cfg, in
         const int64_t ofs = kk * nb, ofst = (kk + 1) * nb;
         const int64_t in = std::min(n - ofs, nb), updm = m - ofs;
         void* p = at(d_a, W, ofs, ofs, ldda);
-        for (int64_t so = 0; so < in; so += x.pw) {
-          const int sw = (int)std::min<int64_t>(x.pw, in - so);
-          const int64_t cm = updm - so, tso = so + sw;
-          RF_CHECK(subpanel_launch(
-              h, W, c.I, true, (int)x.ib, cm, sw, at(p, W, so, so, ldda), ldda,
-              at(p, W, so, so, ldda), ldda,
-              (tc_in || tc_out) ? (half_t*)at(cpy, REMIFA_R_16F, ofs + so, ofs + so, ldc) : nullptr,
-              ldc, x.tab));
-          if (in - tso > 0) {
-            const void* lop = tc_in ? at(cpy, REMIFA_R_16F, ofs + tso, ofs + so, ldc)
-                                    : at(p, W, tso, so, ldda);
-            const void* uop = tc_in ? at(cpy, REMIFA_R_16F, ofs + so, ofs + tso, ldc)
-                                    : at(p, W, so, tso, ldda);
-            const int64_t lop_ld = tc_in ? ldc : ldda;
-            // rank-sw update of the outer block column (:139-163)
-            RF_CHECK(gemm(x, c.I, W, updm - tso, in - tso, sw, lop, lop_ld, uop, lop_ld,
-                          at(p, W, tso, tso, ldda), ldda));
-            // and of the outer block row beyond the outer block (:167-193)
-            if (updm > in) {
-              const void* uop2 = tc_in ? at(cpy, REMIFA_R_16F, ofs + so, ofs + in, ldc)
-                                       : at(p, W, so, in, ldda);
-              RF_CHECK(gemm(x, c.I, W, in - tso, updm - in, sw, lop, lop_ld, uop2, lop_ld,
-                            at(p, W, tso, in, ldda), ldda));
-            }
-          }
-        }
+        RF_CHECK(inner(x, true, W, updm, in, nb, p, ldda, p, ldda,
+                       (tc_in || tc_out) ? at(cpy, REMIFA_R_16F, ofs, ofs, ldc) : nullptr, ldc,
+                       true, p, ldda, ofs));
         // Schur complement (:170-195)
         const int64_t tm = m - ofst, tn = n - ofst;
         if (tn > 0) {
@@ -648,10 +659,7 @@ int lu_nopiv_impl(remifa_handle_t h, int algo, const remifa_lu_config_t* cfg, in
       st = st ? st : REMIFA_ERR_HIP;
   }
   if (st) return st;
-  if (d_info) {
-    info_kernel<<<1, 256, 0, h->stream>>>(n, d_a, ldda, W, d_info);
-    RF_HIP(hipGetLastError());
-  }
+  RF_CHECK(slice_finish_launch(h, W, n, d_a, ldda, ldc, x.pend, d_info));
   // the reference drivers synchronise before returning (:567-569). Under
   // HIP graph capture the call only records its kernels: no readback and no
   // synchronisation (a replay's block-kernel wait flag is then not checked)

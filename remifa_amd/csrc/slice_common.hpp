@@ -1,6 +1,6 @@
-// Shared by the slice kernels (subpanel.hip) and the block kernel
-// (blockll.hip): the arithmetic of the inner factorization and the
-// factorization of a 64 x 64 diagonal tile held in registers.
+// Shared by the slice kernel (slice.hpp) and the block kernel (blockll.hip):
+// the arithmetic of the inner factorization; for the block kernel, the
+// left-looking factorization of a 64 x 64 diagonal tile held in registers.
 #pragma once
 #include <type_traits>
 
@@ -11,11 +11,6 @@ namespace {
 
 constexpr int SW = 64;  // tile edge (slices are at most 64 wide)
 constexpr int PD = 4;   // LDS row padding of the tile
-constexpr int G = 8;    // vector entries held in registers at a time
-
-// published tile: D, D^T, op(D), op(D)^T (64 x 64 row-major each), 1/u_kk, ones
-constexpr int T_D = 0, T_DT = 4096, T_DOP = 8192, T_DOPT = 12288, T_R = 16384, T_ONE = 16448;
-constexpr int T_FLOATS = 16512;
 
 enum SubMode {
   SM_F32 = 0,     // fp32 data, fp32 updates (I = FP32)
@@ -75,8 +70,8 @@ struct Sem {
 // wavefront right of it applies the panel's 8 pivots to its own columns in
 // pivot order. Every entry receives the same sequence of fused updates as in
 // a pivot-by-pivot elimination. ib (a multiple of 8) decides where the block
-// boundaries fall: at a block boundary the block sums (LL: before the block,
-// RL: after it) run as runtime loops over LDS copies of the operands.
+// boundaries fall: at a block boundary the block sums run as runtime loops
+// over LDS copies of the operands.
 constexpr int TP = 8;  // panel width = columns per wavefront
 
 // Row pitches are 16-byte multiples so that a lane publishes its 8 values
@@ -107,7 +102,7 @@ __device__ __forceinline__ float bcast_lane(float v, int lane) {
 // factors (multipliers below the diagonal, U on and above it) and S.R the
 // reciprocals of the pivots. ib is the block size (8, 16, 32 or 64, with
 // SW - ib <= KM).
-template <int MODE, bool RL, int KM>
+template <int MODE, int KM>
 __device__ __forceinline__ void tile_factor(TileLdsT<KM>& S, float (&x)[TP], int ib, int w, int i) {
   using Sm = Sem<MODE>;
   const int cb = w * TP;
@@ -117,7 +112,7 @@ __device__ __forceinline__ void tile_factor(TileLdsT<KM>& S, float (&x)[TP], int
     const int kend = kb + ib;
     // (every wavefront takes every stage: the barrier below needs all eight;
     // columns left of the panel are final and take no work)
-    if (!RL && p0 == kb && kb > 0 && w >= g) {
+    if (p0 == kb && kb > 0 && w >= g) {
       // left-looking update at the start of a block: its columns for the
       // rows >= kb, every column right of it for the rows of the block;
       // products summed from zero in k order, subtracted once
@@ -196,26 +191,8 @@ __device__ __forceinline__ void tile_factor(TileLdsT<KM>& S, float (&x)[TP], int
         for (int jj = 0; jj < TP; ++jj) o[jj] = Sm::op(x[jj]);
         st8(&S.Uo[i][cb], o);
       }
-      if (RL && p0 + TP == kend && cb >= kend) {
-        // block complete: right-looking rank-ib update of the trailing part
-        float acc[TP];
-#pragma unroll
-        for (int jj = 0; jj < TP; ++jj) acc[jj] = 0.0f;
-#pragma unroll 2
-        for (int q = kb; q < kend; ++q) {
-          const float xq = S.Xo[i][q];
-          const float* ur = &S.Uo[q][cb];
-#pragma unroll
-          for (int jj = 0; jj < TP; ++jj) acc[jj] = Sm::acc_add(acc[jj], xq, ur[jj]);
-        }
-        if (i >= kend) {
-#pragma unroll
-          for (int jj = 0; jj < TP; ++jj) x[jj] = Sm::apply(x[jj], acc[jj]);
-        }
-      }
     }
   }
-
 }
 
 }  // namespace
