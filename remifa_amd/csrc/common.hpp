@@ -279,8 +279,6 @@ struct SlicePending {
   int64_t first_col = -1;  // column of the first slice
 };
 
-int copy2d_launch(remifa_handle_t h, size_t elt, int64_t m, int64_t n, const void* a, int64_t lda,
-                  void* b, int64_t ldb);
 
 // device address of the static scratch array of remifa_getrs_nopiv_noalloc
 // on `device` (current), looked up once per device (solve.hip)
