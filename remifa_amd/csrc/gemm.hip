@@ -431,13 +431,12 @@ int split_model(int64_t M, int64_t N, int64_t K, TileGeom tg, int num_cu, double
   return best;
 }
 
-// 256 x 256 tiles on gemm_big_kernel: 16-bit operands in memory, M and N
-// multiples of 256, K a multiple of the 32-deep slab (split-K chunks are
-// multiples of 64), 16-byte aligned operands and column offsets of one slab
-// within 32 bits (the DMA lane offsets)
+// 256 x 256 tiles on gemm_big_kernel: 16-bit operands in memory, M and K in
+// whole 16-byte units (split-K chunks are multiples of 64), 16-byte aligned
+// operands and column offsets of one slab within 32 bits (the DMA lane offsets)
 bool big_fits(int opk, int64_t m, int64_t n, int64_t k, const void* a, int64_t lda, const void* b,
               int64_t ldb) {
-  return (opk == OPK_F16 || opk == OPK_BF16S) && m % 256 == 0 && n % 256 == 0 && k % 32 == 0 &&
+  return (opk == OPK_F16 || opk == OPK_BF16S) && m > 0 && n > 0 && m % 8 == 0 && k % 8 == 0 &&
          (uintptr_t)a % 16 == 0 && (uintptr_t)b % 16 == 0 && lda % 8 == 0 && ldb % 8 == 0 &&
          (64 * lda + 256) * 2 < (int64_t)1 << 31 && (256 * ldb + 64) * 2 < (int64_t)1 << 31;
 }
@@ -447,8 +446,8 @@ bool big_fits(int opk, int64_t m, int64_t n, int64_t k, const void* a, int64_t l
 // matrix-core work (964 -> 1265 TFLOP/s at 8192^3 with eight, MI355X)
 template <int OPK, typename OutT>
 int launch_big(remifa_handle_t h, GemmArgs g, int split) {
-  g.tiles_m = (int)(g.M / 256);
-  g.tiles_n = (int)(g.N / 256);
+  g.tiles_m = (int)ceil_div(g.M, 256);
+  g.tiles_n = (int)ceil_div(g.N, 256);
   dim3 grid((unsigned)(g.tiles_m * g.tiles_n), 1, (unsigned)split);
   gemm_big_kernel<OPK, OutT, 32, 4, 8><<<grid, 512, 0, h->stream>>>(g);
   RF_HIP(hipGetLastError());
@@ -476,9 +475,17 @@ void plan_gemm(remifa_handle_t h, int opk, int64_t m, int64_t n, int64_t K, cons
     return t >= 0 && (opk != OPK_F32 || t == T256x32 || t == T32x256 || t == T128x128);
   };
   if (fits(rule_tile)) tile = rule_tile;  // autotuned table
-  // below K = 2048 the 256 x 256 kernel's start-up and epilogue outweigh its
-  // loop (measured on MI355X at N = 512): 128 x 128 unless forced
-  if (tile == T256x256 && K < 2048) tile = T128x128;
+  // 256 x 256 where its tiles fill the CUs at least once, or K is long enough
+  // for split-K to do so with the start-up and epilogue still small beside the
+  // loop; else 128 x 128, unless forced. Measured (MI355X, us, 128 x 128
+  // against 256 x 256): 8000 x 6000 K = 2000 363 / 221, 4096^2 K = 256 25.6 /
+  // 23.7, 8000^2 K = 512 123 / 100; 2000^2 K = 1024 27 / 32, K = 2048 47 / 42,
+  // K = 4096 66 / 56; 16384 x 512 K = 1024 35 / 39, K = 4096 95 / 87;
+  // 4096 x 512 K = 4096 40 / 50; 1024^2 K = 4096 31 / 34. (The last blocks of
+  // a large LU, 8192 x 512 and less with K above 24000, keep 256 x 256: with
+  // 128 x 128 there n = 32768 took 51.7 ms instead of 50.7.)
+  const int64_t big_tiles = ceil_div(m, 256) * ceil_div(n, 256);
+  if (tile == T256x256 && big_tiles < h->num_cu && K < (big_tiles < 64 ? 8192 : 2048)) tile = T128x128;
   if (fits(h->gemm_tile)) tile = h->gemm_tile;  // explicit override (autotuner runs)
   if (tile == T256x256 && !big_fits(opk, m, n, K, a, lda, b, ldb)) tile = T128x128;
   split = h->split_k > 0 ? h->split_k : rule_split;
@@ -862,6 +869,9 @@ int gemm_launch_cin(remifa_handle_t h, int ctype, int in_t, int out_t, int64_t m
   const int bk = kSplitGranule;
   int tile, split;
   plan_gemm(h, opk, m, n, g.K, a, lda, b, ldb, tile, split);
+  // (the 256 x 256 epilogue's lane offsets into a tile of C are 32 bits)
+  if (tile == T256x256 && 1024 * std::max(ldc, std::max(ldcin, m)) >= (int64_t)1 << 31)
+    tile = T128x128;
   g.kchunk = ceil_div(ceil_div(g.K > 0 ? g.K : 1, split), bk) * bk;
   split = (int)ceil_div(g.K > 0 ? g.K : 1, g.kchunk);
   if (split > 1) {

@@ -33,9 +33,13 @@
 // 512-byte rows of A (two per instruction) or whole BK-element column
 // segments of B, with the 16-byte pieces permuted among the lanes.
 //
-// Shapes: M and N multiples of 256, every K range (K, and the split-K chunk)
-// a multiple of BK, 16-byte aligned operands with leading dimensions that are
-// multiples of 8 (gemm.hip checks, and uses gemm_mfma_kernel otherwise).
+// Shapes: M and K multiples of 8 (whole 16-byte units), any N, 16-byte
+// aligned operands with leading dimensions that are multiples of 8 (gemm.hip
+// checks, and uses gemm_mfma_kernel otherwise). Edge tiles cost the loop
+// nothing: a lane whose rows or columns lie outside the matrix requests the
+// last ones inside it (their products reach only accumulators that are not
+// stored), and a last slab of fewer than BK k-values is cleared beyond them
+// in LDS, in both operands, before it is multiplied.
 
 template <int BK, int WAVES>
 struct BigGeom {
@@ -112,22 +116,32 @@ __global__ void __launch_bounds__(64 * WAVES) gemm_big_kernel(GemmArgs g) {
   const int64_t m0 = (int64_t)tm * 256, n0 = (int64_t)tn * 256;
   const int64_t kbeg = (int64_t)blockIdx.z * g.kchunk;
   const int64_t kend = kbeg + g.kchunk < g.K ? kbeg + g.kchunk : g.K;
-  const int nk = kend > kbeg ? (int)((kend - kbeg) / BK) : 0;
+  const int nk = kend > kbeg ? (int)((kend - kbeg + BK - 1) / BK) : 0;
+  const int ktail = kend > kbeg ? (int)((kend - kbeg) % BK) : 0;  // k-values of a short last slab
+  // rows and columns of C in this tile
+  const int mv = g.M - m0 < 256 ? (int)(g.M - m0) : 256;
+  const int nv = g.N - n0 < 256 ? (int)(g.N - n0) : 256;
 
   const uint16_t* const A = (const uint16_t*)g.A;
   const uint16_t* const B = (const uint16_t*)g.B;
 
-  // DMA lane offsets in bytes from the slab's corner (fixed for the loop)
+  // DMA lane offsets in bytes from the corner of a slab with kv k-values
+  // (fixed for the loop)
   uint32_t offa[LPW], offb[LPW];
+  auto lane_offsets = [&](int kv) {
 #pragma unroll
-  for (int t = 0; t < LPW; ++t) {
-    const int r = wave * (BK / WAVES) + 2 * t + lh;  // A row (k) of this lane
-    const int u = l32 ^ (4 * (r & 3));           // unit loaded into position l32
-    offa[t] = (uint32_t)(((int64_t)r * g.lda + 8 * u) * 2);
-    const int p = (wave * LPW + t) * 64 + lane;  // B position
-    const int n = p / UC, c = (p % UC) ^ ((n / GEO::CPS) % UC);
-    offb[t] = (uint32_t)(((int64_t)n * g.ldb + 8 * c) * 2);
-  }
+    for (int t = 0; t < LPW; ++t) {
+      const int r = wave * (BK / WAVES) + 2 * t + lh;  // A row (k) of this lane
+      const int u = l32 ^ (4 * (r & 3));           // unit loaded into position l32
+      const int ru = r < kv ? r : kv - 1, uu = 8 * u < mv ? u : mv / 8 - 1;
+      offa[t] = (uint32_t)(((int64_t)ru * g.lda + 8 * uu) * 2);
+      const int p = (wave * LPW + t) * 64 + lane;  // B position
+      const int n = p / UC, c = (p % UC) ^ ((n / GEO::CPS) % UC);
+      const int nu = n < nv ? n : nv - 1, cu = 8 * c < kv ? c : kv / 8 - 1;
+      offb[t] = (uint32_t)(((int64_t)nu * g.ldb + 8 * cu) * 2);
+    }
+  };
+  lane_offsets(BK);
   // LDS byte address of the stage area (wave-uniform)
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_vptr)lds);
   auto issue = [&](int k, int st) {
@@ -192,9 +206,14 @@ __global__ void __launch_bounds__(64 * WAVES) gemm_big_kernel(GemmArgs g) {
     }
   };
 
+  // (a short last slab is the last request: its lane offsets replace the others)
+  const int nfull = nk - (ktail != 0);
 #pragma unroll
   for (int p = 0; p < NS - 1; ++p)
-    if (p < nk) issue(p, p);
+    if (p < nk) {
+      if (p == nfull) lane_offsets(ktail);
+      issue(p, p);
+    }
   // steady state: slab k landed while NS - 2 later slabs may be in flight;
   // after slab k is multiplied, slab k + NS - 1 goes into the buffer of slab
   // k - 1 (every wavefront finished that one before the barrier). Requesting
@@ -202,16 +221,33 @@ __global__ void __launch_bounds__(64 * WAVES) gemm_big_kernel(GemmArgs g) {
   // compiler from placing a full vmcnt wait ahead of the fragment reads (it
   // cannot tell the DMA's LDS target from the buffer being read).
   int k = 0, st = 0;
-  for (; k + NS - 1 < nk; ++k) {
+  for (; k + NS - 1 < nfull; ++k) {
     vm_wait_barrier<(NS - 2) * 2 * LPW>();
     compute(st);
     issue(k + NS - 1, st == 0 ? NS - 1 : st - 1);
     st = st == NS - 1 ? 0 : st + 1;
   }
-  // the last NS - 1 slabs: everything requested has to land
+  // the last slabs: everything requested has to land
+  bool short_pending = ktail && nk >= NS;
   for (; k < nk; ++k) {
     vm_wait_barrier<0>();
+    if (k == nfull) {
+      // clear the k-values past the range: whole rows of A, units of B
+      uint16_t* const base = lds + st * GEO::ST;
+      const u16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+      for (int p = ktail * 32 + tid; p < BK * 32; p += 64 * WAVES) *(u16x8*)&base[p * 8] = zero;
+      for (int p = tid; p < 256 * UC; p += 64 * WAVES) {
+        const int n = p / UC, c = (p % UC) ^ ((n / GEO::CPS) % UC);
+        if (8 * c >= ktail) *(u16x8*)&base[GEO::A_ST + p * 8] = zero;
+      }
+      __syncthreads();
+    }
     compute(st);
+    if (short_pending) {
+      lane_offsets(ktail);
+      issue(nfull, st == 0 ? NS - 1 : st - 1);
+      short_pending = false;
+    }
     st = st == NS - 1 ? 0 : st + 1;
   }
 
@@ -225,21 +261,34 @@ __global__ void __launch_bounds__(64 * WAVES) gemm_big_kernel(GemmArgs g) {
     const __amdgpu_buffer_rsrc_t rc =
         __builtin_amdgcn_make_buffer_rsrc(base, 0, 0x7fffffff, kBigBufWord3);
     const uint32_t vo = (uint32_t)((ml + (int64_t)nl * ld) * sizeof(T));
+    auto put = [&](int i, int j, int q) {
+      const uint32_t so =
+          (uint32_t)((32 * i + (int64_t)(32 * j + 8 * (q >> 2) + (q & 3)) * ld) * sizeof(T));
+      const float v = value(i, j, q, so);
+      if constexpr (sizeof(T) == 4)
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rc, vo, so, 0);
+      else
+        __builtin_amdgcn_raw_buffer_store_b16(
+            __builtin_bit_cast(uint16_t, (half_t)v), rc, vo, so, 0);
+    };
+    if (mv == 256 && nv == 256) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int j = 0; j < FN; ++j)
+        for (int j = 0; j < FN; ++j)
 #pragma unroll
-        for (int q = 0; q < 16; ++q) {
-          const uint32_t so =
-              (uint32_t)((32 * i + (int64_t)(32 * j + 8 * (q >> 2) + (q & 3)) * ld) * sizeof(T));
-          const float v = value(i, j, q, so);
-          if constexpr (sizeof(T) == 4)
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rc, vo, so, 0);
-          else
-            __builtin_amdgcn_raw_buffer_store_b16(
-                __builtin_bit_cast(uint16_t, (half_t)v), rc, vo, so, 0);
-        }
+          for (int q = 0; q < 16; ++q) put(i, j, q);
+    } else {
+      // edge tile: rows and columns inside the matrix
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (ml + 32 * i < mv)
+#pragma unroll
+          for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int q = 0; q < 16; ++q)
+              if (nl + 32 * j + 8 * (q >> 2) + (q & 3) < nv) put(i, j, q);
+    }
   };
   if (gridDim.z > 1) {
     // split-K partial alpha * acc of slice z

@@ -30,3 +30,47 @@ def test_half_sums_bitexact(handle, gpu, m, n, k, pad):
     torch.cuda.synchronize()
     ref = orc.f32_to_f16_bits(orc.gemm_sub(orc.FP16, a, b, c, orc.F16))
     assert np.array_equal(to_np(dc), ref)
+
+
+# one tile and a bit in each direction, the smallest, a single column, K of a
+# short slab, below the four stages, around them, and split
+@pytest.mark.parametrize("m,n,k,split", [(8, 1, 8, 1), (264, 255, 40, 1), (248, 257, 24, 1),
+                                         (520, 3, 136, 1), (256, 512, 128, 1),
+                                         (1000, 700, 2008, 1), (272, 300, 1000, 3),
+                                         (8, 600, 200, 2)])
+@pytest.mark.parametrize("out", ["f32", "f16"])
+@pytest.mark.parametrize("beta", [0.0, 1.0])
+def test_big_tile_edges(handle, gpu, m, n, k, split, out, beta):
+    """The 256 x 256 kernel on partial tiles and slabs: within 2 (k + 2) u
+    (|A||B| + |C|) of the FP64 product (any summation order), plus one
+    rounding of an fp16 result, and nothing outside C is touched. What lies
+    beside the operands is NaN and must not reach the result."""
+    import torch
+    import remifa_amd as rf
+    g = torch.Generator().manual_seed(m + 3 * n + k)
+    nan = float("nan")
+    ab = torch.full((k, m + 8), nan, dtype=torch.float16)
+    ab[:, :m] = (torch.rand((k, m), generator=g) - 0.5).half()
+    bb = torch.full((n, k + 16), nan, dtype=torch.float16)
+    bb[:, :k] = (torch.rand((n, k), generator=g) - 0.5).half()
+    dt = torch.float32 if out == "f32" else torch.float16
+    cb = torch.full((n + 2, m + 3), 9.0, dtype=dt)
+    cb[:n, :m] = (torch.rand((n, m), generator=g) - 0.5).to(dt)
+    da, db, dc = ab.to(gpu), bb.to(gpu), cb.to(gpu)
+    handle.set_gemm_tile(4)
+    handle.set_tuning(split_k=split)
+    try:
+        rf.gemmex(handle, rf.TC32, da.t()[:m], db.t()[:k], dc.t()[:m, :n], alpha=-1.0, beta=beta)
+        torch.cuda.synchronize()
+    finally:
+        handle.set_gemm_tile()
+        handle.set_tuning()
+    a, b, c = ab[:, :m].double().t(), bb[:, :k].double().t(), cb[:n, :m].double().t()
+    ref = beta * c - a @ b
+    mag = a.abs() @ b.abs() + beta * c.abs()
+    got = dc.cpu()
+    tol = 2 * (k + 2) * 2.0**-24 * mag
+    if out == "f16":
+        tol = tol + 2.0**-11 * ref.abs() + 2.0**-24
+    assert ((got[:n, :m].double().t() - ref).abs() <= tol).all()
+    assert (got[:, m:] == 9).all() and (got[n:] == 9).all()
