@@ -441,6 +441,23 @@ bool big_fits(int opk, int64_t m, int64_t n, int64_t k, const void* a, int64_t l
          (64 * lda + 256) * 2 < (int64_t)1 << 31 && (256 * ldb + 64) * 2 < (int64_t)1 << 31;
 }
 
+// FP8: 256 x 256 tiles where they fill half the CUs, and for short K whatever
+// the size; between, 128 x 128 tiles (four times the workgroups) hide the
+// latency of a slab better, until K is long enough to split. Lane offsets
+// permitting. Measured (MI355X, us, 128 x 128 against 256 x 256, unsplit):
+// 8192^2 K = 256 101 / 57, K = 4096 533 / 327; 16384 x 512 K = 512 20 / 16,
+// K = 8192 118 / 116; 2048^2 K = 256 15 / 12, K = 1024 21 / 21, K = 2048 30 /
+// 33, K = 8192 87 / 116; 512^2 K = 512 14 / 12, K = 4096 40 / 48.
+int fp8_tile(remifa_handle_t h, int64_t m, int64_t n, int64_t k, const Fp8Args& g) {
+  const int64_t lim = (int64_t)1 << 31;
+  const bool fits = 256 * g.lda + 64 < lim && 256 * g.ldb + 64 < lim && 256 * g.ldsa + 4 < lim &&
+                    256 * g.ldsb + 4 < lim && 1024 * std::max(g.ldc, std::max(g.ldcin, m)) < lim;
+  if (!fits || h->gemm_tile == T128x128) return T128x128;
+  if (h->gemm_tile == T256x256) return T256x256;
+  const int64_t tiles = ceil_div(m, 256) * ceil_div(n, 256);
+  return 2 * tiles >= h->num_cu || k <= 1024 || k >= 16384 ? T256x256 : T128x128;
+}
+
 // 32-deep slabs, four LDS stages (128 KB), eight wavefronts: with four the
 // LDS-DMA requests stalled the one wavefront per SIMD that also issues the
 // matrix-core work (964 -> 1265 TFLOP/s at 8192^3 with eight, MI355X)
@@ -687,25 +704,32 @@ int fp8_quantize_launch(remifa_handle_t h, int in_t, bool rows, int64_t R, int64
   if (ldq % 16 || (uintptr_t)q % 16 || ldq < ceil_div(K, 32) * 32 || lds < ceil_div(K, 32))
     return -7;
   if (ld < (rows ? R : K)) return -5;
-  dim3 grid((unsigned)ceil_div(R, 256), (unsigned)ceil_div(K, 32));
+  if (in_t != REMIFA_R_16F && in_t != REMIFA_R_32F) return -4;
   timer_begin(h, KC_CONVERT, (double)R * K * ((in_t == REMIFA_R_32F ? 4 : 2) + 1), 8);
-  if (in_t == REMIFA_R_16F) {
-    if (rows)
-      quant_fp8_kernel<half_t, true><<<grid, 256, 0, h->stream>>>(R, K, (const half_t*)src, ld, q,
-                                                                  ldq, s, lds);
+  if (rows) {
+    dim3 grid((unsigned)ceil_div(R, 64), (unsigned)ceil_div(K, 128));
+    if (in_t == REMIFA_R_16F)
+      quant_fp8_rows_kernel<half_t>
+          <<<grid, 256, 0, h->stream>>>(R, K, (const half_t*)src, ld, q, ldq, s, lds);
     else
-      quant_fp8_kernel<half_t, false><<<grid, 256, 0, h->stream>>>(R, K, (const half_t*)src, ld,
-                                                                   q, ldq, s, lds);
-  } else if (in_t == REMIFA_R_32F) {
-    if (rows)
-      quant_fp8_kernel<float, true><<<grid, 256, 0, h->stream>>>(R, K, (const float*)src, ld, q,
-                                                                 ldq, s, lds);
-    else
-      quant_fp8_kernel<float, false><<<grid, 256, 0, h->stream>>>(R, K, (const float*)src, ld, q,
-                                                                  ldq, s, lds);
+      quant_fp8_rows_kernel<float>
+          <<<grid, 256, 0, h->stream>>>(R, K, (const float*)src, ld, q, ldq, s, lds);
   } else {
-    timer_end(h);
-    return -4;
+    // threads along K: a power of two between one 32-block and 256
+    int bx = 256;
+    while (bx > 4 && (int64_t)(bx / 2) * 8 >= K) bx /= 2;
+    // (a grid has at most 65535 workgroups along the columns: slices of them)
+    const int64_t cols = (int64_t)(256 / bx) * QC, most = 65535 * cols;
+    for (int64_t c0 = 0; c0 < R; c0 += most) {
+      const int64_t rc = std::min(R - c0, most);
+      dim3 grid((unsigned)ceil_div(K, (int64_t)bx * 8), (unsigned)ceil_div(rc, cols));
+      if (in_t == REMIFA_R_16F)
+        quant_fp8_cols_kernel<half_t><<<grid, dim3(bx, 256 / bx), 0, h->stream>>>(
+            rc, K, (const half_t*)src + c0 * ld, ld, q + c0 * ldq, ldq, s + c0 * lds, lds);
+      else
+        quant_fp8_cols_kernel<float><<<grid, dim3(bx, 256 / bx), 0, h->stream>>>(
+            rc, K, (const float*)src + c0 * ld, ld, q + c0 * ldq, ldq, s + c0 * lds, lds);
+    }
   }
   timer_end(h);
   RF_HIP(hipGetLastError());
@@ -732,13 +756,15 @@ int fp8_gemm_launch(remifa_handle_t h, int out_t, int64_t m, int64_t n, int64_t 
   g.B = qb, g.ldb = ldqb, g.SB = sb, g.ldsb = ldsb;
   g.alpha = alpha, g.beta = beta, g.C = c, g.ldc = ldc;
   g.Cin = cin, g.ldcin = ldcin, g.cin_half = cin_t == REMIFA_R_16F;
-  g.tiles_m = (int)ceil_div(m, 128);
-  g.tiles_n = (int)ceil_div(n, 128);
+  const int tile = fp8_tile(h, m, n, k, g);
+  const int tm = tile == T256x256 ? 256 : 128;
+  g.tiles_m = (int)ceil_div(m, tm);
+  g.tiles_n = (int)ceil_div(n, tm);
   constexpr int BK = 128;
   int split = h->split_k;
   const size_t avail = h->ws_bytes > h->ws_used ? h->ws_bytes - h->ws_used : 0;
   if (split <= 0)
-    split = k > 0 ? split_model(m, n, k, TileGeom{128, 128, 2}, std::max(1, h->num_cu - h->cu_busy),
+    split = k > 0 ? split_model(m, n, k, tile_geom(tile), std::max(1, h->num_cu - h->cu_busy),
                                 7.0e12, BK, avail)
                   : 1;
   g.kchunk = ceil_div(ceil_div(k > 0 ? k : 1, split), BK) * BK;
@@ -752,9 +778,13 @@ int fp8_gemm_launch(remifa_handle_t h, int out_t, int64_t m, int64_t n, int64_t 
     g.W = (float*)((char*)h->ws + h->ws_used);
     g.ldw = m;
   }
-  timer_begin(h, KC_GEMM, 2.0 * (double)m * n * k, (3 << 8) | ((out_t == REMIFA_R_16F) << 4) | T128x128);
+  timer_begin(h, KC_GEMM, 2.0 * (double)m * n * k, (3 << 8) | ((out_t == REMIFA_R_16F) << 4) | tile);
   dim3 grid((unsigned)(g.tiles_m * g.tiles_n), 1, (unsigned)split);
-  if (out_t == REMIFA_R_32F)
+  if (tile == T256x256 && out_t == REMIFA_R_32F)
+    gemm_fp8_big_kernel<float><<<grid, 512, 0, h->stream>>>(g);
+  else if (tile == T256x256)
+    gemm_fp8_big_kernel<half_t><<<grid, 512, 0, h->stream>>>(g);
+  else if (out_t == REMIFA_R_32F)
     gemm_fp8_kernel<float><<<grid, 256, 0, h->stream>>>(g);
   else
     gemm_fp8_kernel<half_t><<<grid, 256, 0, h->stream>>>(g);

@@ -92,6 +92,82 @@ __device__ __forceinline__ void dma16(const u32x4& rsrc, uint32_t voff, uint32_t
                : "memory", "m0");
 }
 
+// epilogue of a 256 x 256 tile at (m0, n0) with mv x nv entries inside the
+// matrix: lane holds C[m = .. + l32][n = .. + 8 (q / 4) + 4 lh + q % 4].
+// Buffer accesses from the tile's corner: a per-lane 32-bit offset (row
+// and lane half) plus a uniform one per (i, j, q), so no 64-bit address
+// arithmetic per element.
+template <typename OutT, int FN, int WTN, typename Args>
+__device__ __forceinline__ void big_epilogue(const Args& g, const f16v (&acc)[4][FN], int wm,
+                                             int wn, int l32, int lh, int64_t m0, int64_t n0,
+                                             int mv, int nv) {
+  const int ml = 128 * wm + l32, nl = WTN * wn + 4 * lh;
+  auto store_all = [&](auto out_tag, void* base, int64_t ld, auto value) {
+    using T = decltype(out_tag);
+    const __amdgpu_buffer_rsrc_t rc =
+        __builtin_amdgcn_make_buffer_rsrc(base, 0, 0x7fffffff, kBigBufWord3);
+    const uint32_t vo = (uint32_t)((ml + (int64_t)nl * ld) * sizeof(T));
+    auto put = [&](int i, int j, int q) {
+      const uint32_t so =
+          (uint32_t)((32 * i + (int64_t)(32 * j + 8 * (q >> 2) + (q & 3)) * ld) * sizeof(T));
+      const float v = value(i, j, q, so);
+      if constexpr (sizeof(T) == 4)
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rc, vo, so, 0);
+      else
+        __builtin_amdgcn_raw_buffer_store_b16(
+            __builtin_bit_cast(uint16_t, (half_t)v), rc, vo, so, 0);
+    };
+    if (mv == 256 && nv == 256) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+          for (int q = 0; q < 16; ++q) put(i, j, q);
+    } else {
+      // edge tile: rows and columns inside the matrix
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (ml + 32 * i < mv)
+#pragma unroll
+          for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int q = 0; q < 16; ++q)
+              if (nl + 32 * j + 8 * (q >> 2) + (q & 3) < nv) put(i, j, q);
+    }
+  };
+  if (gridDim.z > 1) {
+    // split-K partial alpha * acc of slice z
+    float* const wb = g.W + ((int64_t)blockIdx.z * g.N + n0) * g.ldw + m0;
+    store_all(0.0f, (void*)wb, g.ldw,
+              [&](int i, int j, int q, uint32_t) { return g.alpha * acc[i][j][q]; });
+  } else if (g.beta == 0.0f) {
+    store_all(OutT{}, (void*)((OutT*)g.C + m0 + n0 * g.ldc), g.ldc,
+              [&](int i, int j, int q, uint32_t) { return g.alpha * acc[i][j][q]; });
+  } else {
+    // beta term from C itself or from the separate input (fp16 or fp32)
+    const bool half_in = g.Cin ? g.cin_half != 0 : sizeof(OutT) == 2;
+    const void* const cb = g.Cin ? g.Cin : (const void*)g.C;
+    const int64_t ldi = g.Cin ? g.ldcin : g.ldc;
+    const int esz = half_in ? 2 : 4;
+    const __amdgpu_buffer_rsrc_t ri = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)((const char*)cb + (m0 + n0 * ldi) * esz), 0, 0x7fffffff, kBigBufWord3);
+    const uint32_t vi = (uint32_t)((ml + (int64_t)nl * ldi) * esz);
+    store_all(OutT{}, (void*)((OutT*)g.C + m0 + n0 * g.ldc), g.ldc,
+              [&](int i, int j, int q, uint32_t) {
+                const uint32_t si =
+                    (uint32_t)((32 * i + (int64_t)(32 * j + 8 * (q >> 2) + (q & 3)) * ldi) * esz);
+                float c;
+                if (half_in)
+                  c = (float)__builtin_bit_cast(
+                      half_t, (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(ri, vi, si, 0));
+                else
+                  c = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ri, vi, si, 0));
+                return __builtin_fmaf(g.alpha, acc[i][j][q], g.beta * c);
+              });
+  }
+}
+
 template <int OPK, typename OutT, int BK, int NS, int WAVES>
 __global__ void __launch_bounds__(64 * WAVES) gemm_big_kernel(GemmArgs g) {
   using GEO = BigGeom<BK, WAVES>;
@@ -251,73 +327,5 @@ __global__ void __launch_bounds__(64 * WAVES) gemm_big_kernel(GemmArgs g) {
     st = st == NS - 1 ? 0 : st + 1;
   }
 
-  // epilogue: lane holds C[m = .. + l32][n = .. + 8 (q / 4) + 4 lh + q % 4].
-  // Buffer accesses from the tile's corner: a per-lane 32-bit offset (row
-  // and lane half) plus a uniform one per (i, j, q), so no 64-bit address
-  // arithmetic per element.
-  const int ml = 128 * wm + l32, nl = WTN * wn + 4 * lh;
-  auto store_all = [&](auto out_tag, void* base, int64_t ld, auto value) {
-    using T = decltype(out_tag);
-    const __amdgpu_buffer_rsrc_t rc =
-        __builtin_amdgcn_make_buffer_rsrc(base, 0, 0x7fffffff, kBigBufWord3);
-    const uint32_t vo = (uint32_t)((ml + (int64_t)nl * ld) * sizeof(T));
-    auto put = [&](int i, int j, int q) {
-      const uint32_t so =
-          (uint32_t)((32 * i + (int64_t)(32 * j + 8 * (q >> 2) + (q & 3)) * ld) * sizeof(T));
-      const float v = value(i, j, q, so);
-      if constexpr (sizeof(T) == 4)
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rc, vo, so, 0);
-      else
-        __builtin_amdgcn_raw_buffer_store_b16(
-            __builtin_bit_cast(uint16_t, (half_t)v), rc, vo, so, 0);
-    };
-    if (mv == 256 && nv == 256) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-          for (int q = 0; q < 16; ++q) put(i, j, q);
-    } else {
-      // edge tile: rows and columns inside the matrix
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (ml + 32 * i < mv)
-#pragma unroll
-          for (int j = 0; j < FN; ++j)
-#pragma unroll
-            for (int q = 0; q < 16; ++q)
-              if (nl + 32 * j + 8 * (q >> 2) + (q & 3) < nv) put(i, j, q);
-    }
-  };
-  if (gridDim.z > 1) {
-    // split-K partial alpha * acc of slice z
-    float* const wb = g.W + ((int64_t)blockIdx.z * g.N + n0) * g.ldw + m0;
-    store_all(0.0f, (void*)wb, g.ldw,
-              [&](int i, int j, int q, uint32_t) { return g.alpha * acc[i][j][q]; });
-  } else if (g.beta == 0.0f) {
-    store_all(OutT{}, (void*)((OutT*)g.C + m0 + n0 * g.ldc), g.ldc,
-              [&](int i, int j, int q, uint32_t) { return g.alpha * acc[i][j][q]; });
-  } else {
-    // beta term from C itself or from the separate input (fp16 or fp32)
-    const bool half_in = g.Cin ? g.cin_half != 0 : sizeof(OutT) == 2;
-    const void* const cb = g.Cin ? g.Cin : (const void*)g.C;
-    const int64_t ldi = g.Cin ? g.ldcin : g.ldc;
-    const int esz = half_in ? 2 : 4;
-    const __amdgpu_buffer_rsrc_t ri = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)((const char*)cb + (m0 + n0 * ldi) * esz), 0, 0x7fffffff, kBigBufWord3);
-    const uint32_t vi = (uint32_t)((ml + (int64_t)nl * ldi) * esz);
-    store_all(OutT{}, (void*)((OutT*)g.C + m0 + n0 * g.ldc), g.ldc,
-              [&](int i, int j, int q, uint32_t) {
-                const uint32_t si =
-                    (uint32_t)((32 * i + (int64_t)(32 * j + 8 * (q >> 2) + (q & 3)) * ldi) * esz);
-                float c;
-                if (half_in)
-                  c = (float)__builtin_bit_cast(
-                      half_t, (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(ri, vi, si, 0));
-                else
-                  c = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ri, vi, si, 0));
-                return __builtin_fmaf(g.alpha, acc[i][j][q], g.beta * c);
-              });
-  }
+  big_epilogue<OutT, FN, WTN>(g, acc, wm, wn, l32, lh, m0, n0, mv, nv);
 }
