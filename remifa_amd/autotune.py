@@ -137,8 +137,8 @@ def load_rules(path: str = TABLE):
 
 # batched factorization (remifa_lu_nopiv_batched): per size bucket, the
 # thread counts its kernel is built for and the persistent workgroups per CU
-BATCHED = {64: ([64, 128], [2, 4, 8]), 128: ([128, 256], [1, 2, 4]),
-           256: ([256, 512], [1, 2, 3]), 512: ([512], [1, 2])}
+BATCHED = {64: ([64, 128], [2, 4, 8]), 128: ([128, 256], [2, 4, 8]),
+           256: ([256, 512], [1, 2, 4]), 512: ([512], [1, 2])}
 
 
 def tune_batched(count: int = 4000, verbose: bool = True) -> list:

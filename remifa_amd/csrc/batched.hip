@@ -15,11 +15,16 @@
 //  2. the block row U12 = L11^-1 A12, one lane per column;
 //  3. the Schur update A22 -= L21 U12 on the matrix cores from fp16 (bf16)
 //     copies of L21 and U12 staged in LDS, products summed from zero and
-//     subtracted once (the update GEMMs of gemm.hip do the same); four
+//     subtracted once (the update GEMMs of gemm.hip do the same); two
 //     32 x 32 tiles of C per wavefront in flight together.
-// The matrix stays in HBM (the L2 / last-level cache holds it between
-// panels); every element of the trailing matrix is read and written once per
-// panel.
+// The matrix stays in HBM; every element of the trailing matrix is read and
+// written once per panel, which is what bounds orders above 256 (about 7 TB/s
+// over the chip); the pivots and the two triangular steps (25 us per panel of
+// order 500, against 24 us of update) run under another workgroup's update.
+// Measured (MI355X), 2000 matrices of order 257 to 512: 4117 us with one
+// workgroup per CU (80 KB of operands, whole columns read entry by entry in 2.),
+// 3360 with two; 129 to 256: 1139 -> 605 us (four workgroups); 65 to 128: 274 ->
+// 170 us (eight).
 //
 // The batched solve runs one workgroup per matrix: x in LDS, 32-row blocks,
 // the 32x32 diagonal block substitution inside one wavefront, the rest of
@@ -31,24 +36,29 @@ namespace {
 
 constexpr int PW = 32;     // panel width
 constexpr int BMAX = 512;  // largest order
-constexpr int LP = PW + 8; // fp16 row stride of the staged operands (16-byte rows)
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
 
-// LDS of a workgroup for orders up to BM
+// LDS of a workgroup for orders up to BM: 69 KB for 512, so that two
+// workgroups share a CU and one's serial pivots run under the other's updates
 template <int BM>
 struct BatchLds {
-  uint16_t Lh[BM][LP];    // L21 (rows below the panel's top block), fp16/bf16 bits
-  uint16_t Ut[BM][LP];    // U12 transposed: [column][k]
+  uint16_t Lh[BM - PW][PW];  // L21 (rows below the panel's top block), fp16/bf16 bits
+  uint16_t Ut[BM - PW][PW];  // U12 transposed: [column][k]
   __attribute__((aligned(16))) float L11[PW][PW];   // the panel's top block (unit L and U)
   __attribute__((aligned(16))) float L11t[PW][PW];  // its transpose
   float Rk[PW];           // reciprocals of the panel's pivots
   int item;
   int info;
 };
+
+// 16-byte unit c (k-values 8 c .. 8 c + 7) of row r of a staged operand: rows
+// are 64 bytes without padding, units permuted so that the rows of a read
+// phase hit different banks
+__device__ __forceinline__ int unit_at(int r, int c) { return 8 * (c ^ ((r >> 2) & 3)); }
 
 template <bool BF>
 __device__ __forceinline__ uint16_t op_bits(float v) {
@@ -61,7 +71,7 @@ __device__ __forceinline__ uint16_t op_bits(float v) {
 // BM: largest order taken (a size bucket), BT: threads (BT >= BM: one lane
 // per row of a panel and per column of a block row)
 template <bool BF, int BM, int BT>
-__global__ void __launch_bounds__(BT) batched_lu_kernel(int count, const int* __restrict__ d_n,
+__global__ void __launch_bounds__(BT, 4) batched_lu_kernel(int count, const int* __restrict__ d_n,
                                                         const int* __restrict__ d_ld,
                                                         float* const* __restrict__ d_ptrs,
                                                         int* __restrict__ d_info,
@@ -77,7 +87,7 @@ __global__ void __launch_bounds__(BT) batched_lu_kernel(int count, const int* __
       S.info = 0;
     }
     __syncthreads();
-    const int item = S.item;
+    const int item = __builtin_amdgcn_readfirstlane(S.item);  // (uniform addresses below)
     if (item >= count) break;  // every workgroup reaches this: the grid drains
     const int n = d_n[item];
     const int64_t ld = d_ld[item];
@@ -97,7 +107,7 @@ __global__ void __launch_bounds__(BT) batched_lu_kernel(int count, const int* __
 #pragma unroll
         for (int j = 0; j < PW; ++j) {
           const int jc = j < pw ? j : pw - 1;
-          const float v = a[(k0 + r) + (int64_t)(k0 + jc) * ld];
+          const float v = (a + k0 + (int64_t)(k0 + jc) * ld)[(unsigned)r];
           x[j] = (t < mp && j < pw) ? v : (t == j ? 1.0f : 0.0f);
         }
       }
@@ -158,7 +168,7 @@ __global__ void __launch_bounds__(BT) batched_lu_kernel(int count, const int* __
       if (t < mp) {
 #pragma unroll
         for (int j = 0; j < PW; ++j)
-          if (j < pw) a[(k0 + t) + (int64_t)(k0 + j) * ld] = x[j];
+          if (j < pw) (a + k0 + (int64_t)(k0 + j) * ld)[(unsigned)t] = x[j];
       }
       const int mr = n - k0 - pw;  // rows (and columns) of the trailing matrix
       const int mr32 = (mr + 31) & ~31;
@@ -168,7 +178,7 @@ __global__ void __launch_bounds__(BT) batched_lu_kernel(int count, const int* __
 #pragma unroll
         for (int j = 0; j < PW; ++j) v[j / 8][j % 8] = r < mr ? op_bits<BF>(x[j]) : (uint16_t)0;
 #pragma unroll
-        for (int q = 0; q < PW / 8; ++q) *(u16x8*)&S.Lh[r][8 * q] = v[q];
+        for (int q = 0; q < PW / 8; ++q) *(u16x8*)&S.Lh[r][unit_at(r, q)] = v[q];
       }
       __syncthreads();
       if (mr <= 0) continue;
@@ -176,9 +186,8 @@ __global__ void __launch_bounds__(BT) batched_lu_kernel(int count, const int* __
       if (t < mr32) {
         const int c = t < mr ? t : mr - 1;
         float* col = a + k0 + (int64_t)(k0 + pw + c) * ld;
-        float u[PW];
-#pragma unroll
-        for (int i = 0; i < PW; ++i) u[i] = col[i];
+        float u[PW];  // (the column's 128 bytes as 16-byte accesses, element-aligned)
+        __builtin_memcpy(u, col, sizeof(u));
 #pragma unroll
         for (int kk = 0; kk < PW; ++kk) {
           {
@@ -193,21 +202,18 @@ __global__ void __launch_bounds__(BT) batched_lu_kernel(int count, const int* __
             for (int i = kk + 1; i < PW; ++i) u[i] = __builtin_fmaf(-lc[i], u[kk], u[i]);
           }
         }
-        if (t < mr) {
-#pragma unroll
-          for (int i = 0; i < PW; ++i) col[i] = u[i];
-        }
+        if (t < mr) __builtin_memcpy(col, u, sizeof(u));
         u16x8 v[PW / 8];
 #pragma unroll
         for (int i = 0; i < PW; ++i) v[i / 8][i % 8] = t < mr ? op_bits<BF>(u[i]) : (uint16_t)0;
 #pragma unroll
-        for (int q = 0; q < PW / 8; ++q) *(u16x8*)&S.Ut[t][8 * q] = v[q];
+        for (int q = 0; q < PW / 8; ++q) *(u16x8*)&S.Ut[t][unit_at(t, q)] = v[q];
       }
       __syncthreads();
-      // ---- 3. A22 -= L21 U12 on the matrix cores, 32 x 32 tiles, up to four
-      // per wavefront at a time (their C entries read in one round trip)
+      // ---- 3. A22 -= L21 U12 on the matrix cores, 32 x 32 tiles, two per
+      // wavefront at a time (their C entries read in one round trip)
       const int nt = mr32 / 32;
-      constexpr int TQ = 4;
+      constexpr int TQ = 2;
       for (int tile0 = wave; tile0 < nt * nt; tile0 += TQ * (BT / 64)) {
         f16v acc[TQ];
         float cv[TQ][16];
@@ -227,8 +233,9 @@ __global__ void __launch_bounds__(BT) batched_lu_kernel(int count, const int* __
           for (int q = 0; q < 16; ++q) acc[z][q] = 0.0f;
 #pragma unroll
           for (int ks = 0; ks < PW; ks += 16) {
-            const u16x8 xb = *(const u16x8*)&S.Ut[tn * 32 + l32][ks + 8 * lh];
-            const u16x8 ya = *(const u16x8*)&S.Lh[tm * 32 + l32][ks + 8 * lh];
+            const int rb = tn * 32 + l32, ra = tm * 32 + l32, c = ks / 8 + lh;
+            const u16x8 xb = *(const u16x8*)&S.Ut[rb][unit_at(rb, c)];
+            const u16x8 ya = *(const u16x8*)&S.Lh[ra][unit_at(ra, c)];
             if constexpr (BF)
               acc[z] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
                   __builtin_bit_cast(bf8, xb), __builtin_bit_cast(bf8, ya), acc[z], 0, 0, 0);
@@ -260,8 +267,23 @@ __global__ void __launch_bounds__(BT) batched_lu_kernel(int count, const int* __
   }
 }
 
-// One matrix per workgroup: b <- (L U)^-1 b with the factors in place.
-__global__ void __launch_bounds__(256) batched_getrs_kernel(int count, const int* __restrict__ d_n,
+// lane k's value in every lane
+__device__ __forceinline__ float lane_value(float v, int k) {
+  return __builtin_bit_cast(float,
+                            __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), k));
+}
+
+// One matrix per workgroup: b <- (L U)^-1 b with the factors in place. Bound by
+// the latency of a 32-column step (a read of the factors, the substitution, two
+// barriers): the step's entries of the factors, which do not depend on the
+// solution, are all requested before the substitution, NV rows of the update
+// per thread. BT threads and NV for the caller's largest order (64 threads up
+// to 64, 256 and one row up to 288, else two rows); an order above it still
+// takes the remaining rows one by one. Measured (MI355X), 2000 matrices of
+// order 257 to 512: 739 -> 375 us; 129 to 256: 285 -> 121 us; 16 to
+// 64: 25 -> 19 us.
+template <int BT, int NV>
+__global__ void __launch_bounds__(BT) batched_getrs_kernel(int count, const int* __restrict__ d_n,
                                                             const int* __restrict__ d_ld,
                                                             float* const* __restrict__ d_ptrs,
                                                             float* const* __restrict__ d_b) {
@@ -273,65 +295,81 @@ __global__ void __launch_bounds__(256) batched_getrs_kernel(int count, const int
   const float* __restrict__ a = d_ptrs[item];
   float* __restrict__ b = d_b[item];
   const int t = threadIdx.x;
-  for (int i = t; i < n; i += 256) xs[i] = b[i];
+  for (int i = t; i < n; i += BT) xs[i] = b[i];
   __syncthreads();
+  // row i (in bounds) of the columns k0 .. k0 + kw - 1, the last repeated
+  auto read_row = [&](int i, int k0, int kw, float (&w)[32]) {
+#pragma unroll
+    for (int k = 0; k < 32; ++k) w[k] = (a + (int64_t)(k0 + (k < kw ? k : kw - 1)) * ld)[(unsigned)i];
+  };
+  // x_i -= the row's products with x_k0 .. in order
+  auto update = [&](int i, int k0, int kw, const float (&w)[32]) {
+    float s = xs[i];
+#pragma unroll
+    for (int k = 0; k < 32; ++k)
+      if (k < kw) s = __builtin_fmaf(-w[k], xs[k0 + k], s);
+    xs[i] = s;
+  };
+  float rowv[32], w0[32], w1[32];  // (w1: two rows per thread)
   // forward: unit lower L
   for (int k0 = 0; k0 < n; k0 += 32) {
     const int kw = n - k0 < 32 ? n - k0 : 32;
+    const int i0 = k0 + kw + t, below = n - k0 - kw;
+    if (t < 64) read_row(k0 + (t < kw ? t : 0), k0, kw, rowv);
+    if (t < below) read_row(i0, k0, kw, w0);
+    if (NV == 2 && t + BT < below) read_row(i0 + BT, k0, kw, w1);
     if (t < 64) {
-      // the diagonal block inside one wavefront (lanes 0..kw-1 own its rows;
-      // the lane's row of the block is read before the substitution)
-      const int tr = t < kw ? t : 0;
-      float rowv[32];
-#pragma unroll
-      for (int k = 0; k < 32; ++k) rowv[k] = a[(k0 + tr) + (int64_t)(k0 + (k < kw ? k : 0)) * ld];
+      // the diagonal block inside one wavefront (lanes 0..kw-1 own its rows)
       float xi = t < kw ? xs[k0 + t] : 0.0f;
 #pragma unroll
       for (int k = 0; k < 32; ++k) {
         if (k < kw) {
-          const float xk = __shfl(xi, k, 64);
+          const float xk = lane_value(xi, k);
           if (t > k && t < kw) xi = __builtin_fmaf(-rowv[k], xk, xi);
         }
       }
       if (t < kw) xs[k0 + t] = xi;
     }
     __syncthreads();
-    for (int i = k0 + kw + t; i < n; i += 256) {
-      float s = xs[i];
-      for (int k = 0; k < kw; ++k) s = __builtin_fmaf(-a[i + (int64_t)(k0 + k) * ld], xs[k0 + k], s);
-      xs[i] = s;
-    }
+    if (t < below) update(i0, k0, kw, w0);
+    if (NV == 2 && t + BT < below) update(i0 + BT, k0, kw, w1);
+    if constexpr (BT * NV < BMAX)
+      for (int i = i0 + BT * NV; i < n; i += BT) {
+        read_row(i, k0, kw, w0);
+        update(i, k0, kw, w0);
+      }
     __syncthreads();
   }
   // backward: upper U
   for (int k1 = n; k1 > 0; k1 -= 32) {
     const int k0 = k1 - 32 > 0 ? k1 - 32 : 0;
     const int kw = k1 - k0;
+    if (t < 64) read_row(k0 + (t < kw ? t : 0), k0, kw, rowv);
+    if (t < k0) read_row(t, k0, kw, w0);
+    if (NV == 2 && t + BT < k0) read_row(t + BT, k0, kw, w1);
     if (t < 64) {
-      const int tr = t < kw ? t : 0;
-      float rowv[32];
-#pragma unroll
-      for (int k = 0; k < 32; ++k) rowv[k] = a[(k0 + tr) + (int64_t)(k0 + (k < kw ? k : 0)) * ld];
       float xi = t < kw ? xs[k0 + t] : 0.0f;
 #pragma unroll
       for (int k = 31; k >= 0; --k) {
         if (k < kw) {
           if (t == k) xi = xi / rowv[k];
-          const float xk = __shfl(xi, k, 64);
+          const float xk = lane_value(xi, k);
           if (t < k) xi = __builtin_fmaf(-rowv[k], xk, xi);
         }
       }
       if (t < kw) xs[k0 + t] = xi;
     }
     __syncthreads();
-    for (int i = t; i < k0; i += 256) {
-      float s = xs[i];
-      for (int k = 0; k < kw; ++k) s = __builtin_fmaf(-a[i + (int64_t)(k0 + k) * ld], xs[k0 + k], s);
-      xs[i] = s;
-    }
+    if (t < k0) update(t, k0, kw, w0);
+    if (NV == 2 && t + BT < k0) update(t + BT, k0, kw, w1);
+    if constexpr (BT * NV < BMAX)
+      for (int i = t + BT * NV; i < k0; i += BT) {
+        read_row(i, k0, kw, w0);
+        update(i, k0, kw, w0);
+      }
     __syncthreads();
   }
-  for (int i = t; i < n; i += 256) b[i] = xs[i];
+  for (int i = t; i < n; i += BT) b[i] = xs[i];
 }
 
 __global__ void zero_queue_kernel(int* q) {
@@ -408,8 +446,8 @@ extern "C" int remifa_lu_nopiv_batched(remifa_handle_t h, int ctype, int64_t cou
 // Threads and workgroups per CU of the batched factorization for orders up
 // to bm: the handle's table (remifa_set_batched_tuning) or the defaults.
 void remifa::batched_shape(remifa_handle_t h, int bm, int* bt, int* per_cu) {
-  *bt = bm < 128 ? 128 : (bm < 512 ? 256 : 512);
-  *per_cu = bm <= 64 ? 4 : (bm <= 128 ? 4 : (bm <= 256 ? 2 : 1));
+  *bt = bm;
+  *per_cu = bm <= 128 ? 8 : (bm <= 256 ? 4 : 2);
   for (const auto& r : h->batched_rules)
     if (r[0] == bm) {
       *bt = r[1];
@@ -426,7 +464,13 @@ extern "C" int remifa_getrs_nopiv_batched(remifa_handle_t h, int64_t count, cons
   if (max_n < 0 || max_n > BMAX) return -7;
   if (count == 0) return 0;
   timer_begin(h, KC_OTHER, 0.0, 2);
-  batched_getrs_kernel<<<(unsigned)count, 256, 0, h->stream>>>((int)count, d_n, d_ld, d_ptrs, d_b);
+  const unsigned grid = (unsigned)count;
+  if (max_n <= 64)
+    batched_getrs_kernel<64, 1><<<grid, 64, 0, h->stream>>>((int)count, d_n, d_ld, d_ptrs, d_b);
+  else if (max_n <= 288)
+    batched_getrs_kernel<256, 1><<<grid, 256, 0, h->stream>>>((int)count, d_n, d_ld, d_ptrs, d_b);
+  else
+    batched_getrs_kernel<256, 2><<<grid, 256, 0, h->stream>>>((int)count, d_n, d_ld, d_ptrs, d_b);
   timer_end(h);
   RF_HIP(hipGetLastError());
   return 0;
