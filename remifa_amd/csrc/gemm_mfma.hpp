@@ -14,7 +14,11 @@
 //    multiples of the 16-byte chunk) load whole chunks: a chunk is either in
 //    range or replaced by zeros through an address clamp and a select, so
 //    the loop body has no branches and the prefetch stays asynchronous.
-//    Other shapes use the element-wise VEC = false instantiation.
+//    Other shapes and alignments (VEC = false) read chunks at element
+//    alignment: rows and columns outside the matrix repeat its last ones, and
+//    only a last slab that a chunk could leave A or the K range in goes element
+//    by element. Measured (MI355X): the updates of an n = 5001 fp16 LU with an
+//    odd leading dimension 617 us, 1301 with every chunk element by element.
 //  * A slabs are stored m-contiguous ([k][m]) and B slabs k-contiguous
 //    ([n][k]), both with 16-byte stores; a B fragment is one 16-byte LDS
 //    read, an A fragment (fp16/bf16) two LDS transpose reads.
@@ -26,6 +30,9 @@ typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+// the same chunks at any element address
+typedef uint16_t u16x8u __attribute__((ext_vector_type(8), aligned(2)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef short v4i16 __attribute__((ext_vector_type(4)));
 typedef uint16_t v4u16 __attribute__((ext_vector_type(4)));
 
@@ -88,6 +95,7 @@ struct OpTraits<OPK_F16> {
   using Lds = uint16_t;  // element in LDS
   static constexpr int CH = 8;  // elements per 16-byte chunk
   using Chunk = u16x8;
+  using ChunkU = u16x8u;
   static __device__ __forceinline__ Chunk cvt(Chunk c) { return c; }
 };
 template <>
@@ -96,6 +104,7 @@ struct OpTraits<OPK_BF16> {
   using Lds = uint16_t;
   static constexpr int CH = 8;
   using Chunk = u16x8;
+  using ChunkU = u16x8u;
   // fp16 storage -> bf16 operand, round to nearest even
   static __device__ __forceinline__ Chunk cvt(Chunk c) {
     Chunk r;
@@ -113,6 +122,7 @@ struct OpTraits<OPK_BF16S> {
   using Lds = uint16_t;
   static constexpr int CH = 8;
   using Chunk = u16x8;
+  using ChunkU = u16x8u;
   static __device__ __forceinline__ Chunk cvt(Chunk c) { return c; }
 };
 template <>
@@ -121,6 +131,7 @@ struct OpTraits<OPK_F32> {
   using Lds = float;
   static constexpr int CH = 4;
   using Chunk = f32x4;
+  using ChunkU = f32x4u;
   static __device__ __forceinline__ Chunk cvt(Chunk c) { return c; }
 };
 
@@ -156,6 +167,7 @@ __device__ __forceinline__ void gemm_mfma_body(const GemmArgs& g, int bid, int b
   using S = typename TR::Store;
   using L = typename TR::Lds;
   using Chunk = typename TR::Chunk;
+  using ChunkL = std::conditional_t<VEC, Chunk, typename TR::ChunkU>;  // in memory
   constexpr int CH = TR::CH;
   constexpr int WTM = BM / WM, WTN = BN / WN;
   constexpr int FM = WTM / 32, FN = WTN / 32;
@@ -205,35 +217,44 @@ __device__ __forceinline__ void gemm_mfma_body(const GemmArgs& g, int bid, int b
   // plus per-lane 32-bit element offsets fixed for the whole loop
   const S* const At = A + m0 + kbeg * g.lda;
   const S* const Bt = B + kbeg + n0 * g.ldb;
+  // (VEC = false: the chunk holding the last row, the last column, instead of
+  // those outside the matrix; their products are not stored)
   uint32_t offa[NA], offb[NB];
+  const int mlast = g.M - m0 < BM ? (int)((g.M - m0 - 1) / CH) * CH : BM;
+  const int nlast = g.N - n0 < BN ? (int)(g.N - n0 - 1) : BN;
 #pragma unroll
   for (int p = 0; p < NA; ++p) {
     const int c = tid + 256 * p;
-    offa[p] = (uint32_t)((c % (BM / CH)) * CH + (int64_t)(c / (BM / CH)) * g.lda);
+    int mq = (c % (BM / CH)) * CH;
+    if (!VEC) mq = mq < mlast ? mq : mlast;
+    offa[p] = (uint32_t)(mq + (int64_t)(c / (BM / CH)) * g.lda);
   }
 #pragma unroll
   for (int p = 0; p < NB; ++p) {
     const int c = tid + 256 * p;
-    offb[p] = (uint32_t)((c % (BK / CH)) * CH + (int64_t)(c / (BK / CH)) * g.ldb);
+    int n = c / (BK / CH);
+    if (!VEC) n = n < nlast ? n : nlast;
+    offb[p] = (uint32_t)((c % (BK / CH)) * CH + (int64_t)n * g.ldb);
   }
 
-  // FULL (a tag type): every slab of this tile is in range, so the loads
-  // need no address clamps and the stores no zero-selects
+  // FULL (a tag type): every chunk of the slab is in range (as offa, offb
+  // have it), so the loads need no address clamps and the stores no
+  // zero-selects
   auto load_slab = [&](int kt, auto full_tag) {
     constexpr bool FULL = decltype(full_tag)::value;
     const int64_t kk0 = kbeg + (int64_t)kt * BK;
-    if constexpr (VEC && FULL) {
+    if constexpr (FULL) {
       const S* const as = At + (int64_t)kt * BK * g.lda;
       const S* const bs = Bt + (int64_t)kt * BK;
 #pragma unroll
       for (int p = 0; p < NA; ++p) {
         if (TA % 256 && tid + 256 * p >= TA) break;
-        ra[p] = *(const Chunk*)(as + offa[p]);
+        ra[p] = *(const ChunkL*)(as + offa[p]);
       }
 #pragma unroll
       for (int p = 0; p < NB; ++p) {
         if (TB % 256 && tid + 256 * p >= TB) break;
-        rb[p] = *(const Chunk*)(bs + offb[p]);
+        rb[p] = *(const ChunkL*)(bs + offb[p]);
       }
       return;
     }
@@ -397,13 +418,41 @@ __device__ __forceinline__ void gemm_mfma_body(const GemmArgs& g, int bid, int b
       __syncthreads();
     }
   };
-  // interior tiles (the bulk of the LU's updates) take the unmasked loop
-  // (when the lane offsets above fit in 32 bits)
-  if (VEC && m0 + BM <= g.M && n0 + BN <= g.N && klen % BK == 0 &&
-      (int64_t)BK * g.lda < (1LL << 31) && (int64_t)BN * g.ldb < (1LL << 31))
-    run(std::integral_constant<bool, true>{});
-  else
-    run(std::integral_constant<bool, false>{});
+  const bool off32 = (int64_t)BK * g.lda < (1LL << 31) && (int64_t)BN * g.ldb < (1LL << 31);
+  if constexpr (VEC) {
+    // interior tiles (the bulk of the LU's updates) take the unmasked loop
+    // (when the lane offsets above fit in 32 bits)
+    if (m0 + BM <= g.M && n0 + BN <= g.N && klen % BK == 0 && off32)
+      run(std::integral_constant<bool, true>{});
+    else
+      run(std::integral_constant<bool, false>{});
+  } else {
+    // A chunk past the last row reads on into the next column, except in A's
+    // last column; a short slab's chunks would leave the K range: that slab is
+    // masked (lda >= CH keeps the last column but one inside A)
+    const bool mask_last =
+        klen % BK != 0 || (kend == g.K && g.M % CH != 0 && m0 + BM >= g.M);
+    const int nfull = !(off32 && g.lda >= CH) ? 0 : (mask_last ? nk - 1 : nk);
+    auto load = [&](int kt) {
+      if (kt < nfull)
+        load_slab(kt, std::integral_constant<bool, true>{});
+      else
+        load_slab(kt, std::integral_constant<bool, false>{});
+    };
+    if (nk > 0) {
+      load(0);
+      store_tiles(0, std::integral_constant<bool, true>{});
+    }
+    __syncthreads();
+    for (int kt = 0; kt < nk; ++kt) {
+      const int buf = kt & 1;
+      const bool more = kt + 1 < nk;
+      if (more) load(kt + 1);
+      compute(buf);
+      if (more) store_tiles(buf ^ 1, std::integral_constant<bool, true>{});
+      __syncthreads();
+    }
+  }
 
   // epilogue: lane holds C[m = .. + l32][n = .. + 8*(q/4) + 4*lh + q%4]
 #pragma unroll

@@ -74,3 +74,45 @@ def test_big_tile_edges(handle, gpu, m, n, k, split, out, beta):
         tol = tol + 2.0**-11 * ref.abs() + 2.0**-24
     assert ((got[:n, :m].double().t() - ref).abs() <= tol).all()
     assert (got[:, m:] == 9).all() and (got[n:] == 9).all()
+
+
+# element-aligned operands: rows and K around the 8 (4) of a chunk, the tiles'
+# edges, K around a slab, a leading dimension below a chunk, split
+@pytest.mark.parametrize("m,n,k,pad,split", [(1, 1, 1, 0, 1), (3, 5, 200, 0, 1), (9, 31, 64, 1, 1),
+                                             (33, 257, 63, 3, 1), (129, 127, 129, 0, 1),
+                                             (255, 33, 128, 1, 1), (257, 130, 1000, 2, 3),
+                                             (301, 299, 256, 1, 1)])
+@pytest.mark.parametrize("ctype", ["TC32", "BF16_TC32", "FP32"])
+@pytest.mark.parametrize("tile", [0, 1, 5])
+def test_unaligned_operands(handle, gpu, m, n, k, pad, split, ctype, tile):
+    """Within 2 (k + 2) u (|A||B| + |C|) of the FP64 product of the rounded
+    operands; the padding is NaN and must not reach the result. The operands
+    start at an odd element."""
+    import torch
+    import remifa_amd as rf
+    g = torch.Generator().manual_seed(m + 3 * n + k)
+    dt = torch.float32 if ctype == "FP32" else torch.float16
+
+    def operand(r, c):  # r x c column-major, ld r + pad, NaN beside it
+        buf = torch.full((1 + c * (r + pad),), float("nan"), dtype=dt)
+        v = buf[1:].view(c, r + pad).t()[:r]
+        v.copy_((torch.rand((r, c), generator=g) - 0.5).to(dt))
+        return v.double(), buf.to(gpu)[1:].view(c, r + pad).t()[:r]
+    a, da = operand(m, k)
+    b, db = operand(k, n)
+    if ctype == "BF16_TC32":
+        a, b = a.bfloat16().double(), b.bfloat16().double()
+    c = torch.rand((n, m + 1), generator=g) - 0.5
+    dc = c.to(gpu)
+    handle.set_gemm_tile(tile)
+    handle.set_tuning(split_k=split)
+    try:
+        rf.gemmex(handle, getattr(rf, ctype), da, db, dc.t()[:m], alpha=-1.0, beta=1.0)
+        torch.cuda.synchronize()
+    finally:
+        handle.set_gemm_tile()
+        handle.set_tuning()
+    c64 = c[:, :m].double().t()
+    tol = 2 * (k + 2) * 2.0**-24 * (a.abs() @ b.abs() + c64.abs())
+    assert ((dc.cpu()[:, :m].double().t() - (c64 - a @ b)).abs() <= tol).all()
+    assert torch.equal(dc.cpu()[:, m:], c[:, m:])
