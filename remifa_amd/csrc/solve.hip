@@ -39,7 +39,7 @@ namespace {
 constexpr int NBS = 128;     // block size of the triangular solves
 constexpr int TT = 4 * NBS;  // threads of a triangular-solve workgroup
 constexpr int QC = NBS / 4;  // columns of a block per lane (column quarter)
-constexpr int RC = 16;   // right-hand sides per launch
+constexpr int RC = 16;       // right-hand sides of a group
 constexpr long long kSpinLimit = 1LL << 22;  // retries of a wait (each a memory round trip)
 
 template <typename LT>
