@@ -2,12 +2,14 @@
 // fp32 accumulation; included by gemm.hip inside its anonymous namespace,
 // after gemm_mfma.hpp (GemmArgs, xcd_tile, c_in16, ds_read_tr16).
 //
-// One 256-thread workgroup (four wave64s in 2 x 2) owns a 256 x 256 tile of
-// C, each wavefront a 128 x 128 sub-tile of 4 x 4 v_mfma_f32_32x32x16 blocks
-// (256 fp32 accumulators per lane, one workgroup per CU). Against the
-// 128 x 128 tile of gemm_mfma_kernel (64 x 64 per wavefront) this halves both
-// the operand bytes a CU pulls from L2 per flop and the LDS fragment reads
-// per matrix-core instruction (8 fragments per 16 instructions).
+// One 512-thread workgroup (eight wave64s in 2 x 4) owns a 256 x 256 tile of
+// C, each wavefront a 128 x 64 sub-tile of 4 x 2 v_mfma_f32_32x32x16 blocks
+// (128 fp32 accumulators per lane, one workgroup per CU). Against the
+// 128 x 128 tile of gemm_mfma_kernel (64 x 64 per wavefront) this halves the
+// operand bytes a CU pulls from L2 per flop; per 32-deep slab the LDS (fragment
+// reads and arriving slabs) and the matrix cores are busy 1024 cycles each.
+// Measured (MI355X): 8192^3 949 us (1.16 PFLOP/s), 8000 x 6000 x 2000 201 us
+// (128 x 128 tiles: 1330 and 328 us).
 //
 // Operand slabs go from global memory straight into LDS, without staging
 // registers: buffer_load_dwordx4 ... lds writes each lane's 16 bytes at the
