@@ -634,21 +634,35 @@ __global__ void __launch_bounds__(TT) trsm16_kernel(int64_t n, int nrhs, int ngr
     acc = product(tv, xs[q & 1], acc);
   }
   float* const xr = xs[nsteps & 1];
+  bool finite = true;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int rr = 16 * w + 4 * lq + j;
-    xr[(rr % KS) * XP + (rr / KS) * RC + l16] = bv[j] - acc[j];
+    const float v = bv[j] - acc[j];
+    xr[(rr % KS) * XP + (rr / KS) * RC + l16] = v;
+    finite &= __builtin_isfinite(v);
   }
   __syncthreads();
-  f4v y = product(dv, xr, (f4v){0.0f, 0.0f, 0.0f, 0.0f});
+  f4v y = product(dv, xr, (f4v){0.0f, 0.0f, 0.0f, 0.0f}), yd = y;
+  if (__ballot(!finite) != 0) {
+    // an infinite entry times the diagonal's place, now zero, is NaN: where
+    // an entry is not finite its row takes the product with the diagonal in it
+    const float d0 = inv[((int64_t)bi * NBS + 16 * w + l16) * NBS + 16 * w + l16];
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+      if (32 * lq + s == 16 * w + l16) dv[s] = d0;
+    yd = product(dv, xr, (f4v){0.0f, 0.0f, 0.0f, 0.0f});
+  }
+  f4v z = {0.0f, 0.0f, 0.0f, 0.0f};
   if (fold) {
     float* const xn = xs[(nsteps + 1) & 1];
     stage(tk - 1, xn);
-    y -= product(mv, xn, (f4v){0.0f, 0.0f, 0.0f, 0.0f});
+    z = product(mv, xn, z);
   }
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    y[j] = __builtin_fmaf(dd[j], bv[j] - acc[j], y[j]);
+    const float v = bv[j] - acc[j];
+    y[j] = __builtin_isfinite(v) ? __builtin_fmaf(dd[j], v, y[j] - z[j]) : yd[j] - z[j];
     if (go + j < n && l16 < nr) {
       __hip_atomic_store(&tags[go + j + (int64_t)l16 * n],
                          (1ull << 32) | (unsigned long long)__float_as_uint(y[j]),
