@@ -11,8 +11,8 @@
 // of ib, default 64): each slice is one launch (slice.hip) that subtracts the
 // earlier slices of the outer block (LL: one sum; RL: slice by slice, as the
 // rank-pw updates after each slice would) and does the reference's ib loop.
-// fp16-accumulated sums, and bf16 ones of fp32 buffers, come from update
-// GEMMs between the slices instead. pw = ib reproduces the reference's
+// fp16-accumulated sums, bf16 ones of fp32 buffers and those of wide outer
+// blocks come from update GEMMs between the slices instead. pw = ib reproduces the reference's
 // structure of one panel per ib columns.
 //
 // Differences from the reference, all deliberate:
@@ -75,13 +75,40 @@ size_t gemm_reserve(int64_t m, int64_t nb) {
   return std::min<size_t>((size_t)256 << 20, std::max<size_t>((size_t)16 << 20, full));
 }
 
+// fp16 storage factored in fp32 buffers of one block column and block row
+bool buffered_layout(int algo, const remifa_lu_config_t& c) {
+  return algo == REMIFA_LL && c.W == REMIFA_R_16F && c.IP == REMIFA_R_32F;
+}
+
+// Bytes of the slices' operand copies, or 0 where the updates between the
+// slices are GEMMs instead: in types the slice kernel has no sums for, where
+// the copies (of an outer block w = min(nb, m) wide) would exceed 1 GiB, and in
+// wide outer blocks, whose sums are faster as GEMMs of the whole chip:
+// right-looking (one sum per earlier slice, each a round trip), fp32 (its
+// matrix rate) and, wider still, fp16 operands. Measured (MI355X, ms, sums in
+// the slices against GEMMs): right-looking n = 2048 fp32 nb = 512 1.38 / 1.47,
+// 768 1.67 / 1.48, 2048 3.81 / 1.16; left-looking n = 8192 fp32 nb = 1024 9.0 /
+// 11.0, 2048 12.1 / 11.8, 4096 19.0 / 13.2; fp16 operands nb = 1024 4.4 / 6.3,
+// 4608 8.8 / 8.0, 8192 15.2 / 12.8. bf16 operands read as they are rounded are
+// faster in the slices at every width (nb = 8192 15.5 / 33).
+size_t slice_sum_bytes(int algo, const remifa_lu_config_t& c, int64_t m, int64_t nb) {
+  const int T = buffered_layout(algo, c) ? REMIFA_R_32F : c.W;
+  const int64_t w = std::min(nb, m);
+  const int64_t most = algo == REMIFA_RL        ? 512
+                       : c.I == REMIFA_FP32     ? 1024
+                       : c.I == REMIFA_BF16_TC32 ? w
+                                                : 4096;
+  if (!slice_updates(T, c.I) || w > most) return 0;
+  const size_t b = slice_op_bytes(T, c.I, m, w);
+  return b <= (size_t)1 << 30 ? b : 0;
+}
+
 // the handle stream's part of the arena past the fixed areas: the split-K
 // partials of its update GEMMs and, while it runs the slices of an outer
 // block (no split-K update runs on that stream then), the slices' operand
-// copies
-size_t main_reserve(const remifa_lu_config_t& c, int T, int64_t m, int64_t nb) {
-  const size_t op = slice_updates(T, c.I) ? slice_op_bytes(T, c.I, m, nb) : 0;
-  return std::max(gemm_reserve(m, nb), op);
+// copies (sums bytes)
+size_t main_reserve(int64_t m, int64_t nb, size_t sums) {
+  return std::max(gemm_reserve(m, nb), sums);
 }
 
 struct Ctx {
@@ -89,7 +116,7 @@ struct Ctx {
   remifa_lu_config_t c;
   int64_t ib;
   int pw;             // slice width of the inner factorization
-  void* ops;          // the slices' operand copies
+  void* ops;          // the slices' operand copies (null: GEMMs between the slices)
   SlicePending pend;  // the last slice's tile
 };
 
@@ -115,11 +142,12 @@ inline void* at(void* p, int t, int64_t i, int64_t j, int64_t ld) {
 int inner(Ctx& x, bool rl, int T, int64_t m, int64_t n, int64_t nb, void* l, int64_t ldl, void* u,
           int64_t ldu, void* cpy, int64_t ldcp, bool store_x, void* a, int64_t lda, int64_t col) {
   const int I = x.c.I, W = x.c.W;
-  // update GEMMs between the slices where the slice kernel has no sums for
-  // the type; with T = fp32 and an inner TC type their operands are read
-  // from the mirror
-  const bool ext = !slice_updates(T, I);
+  // update GEMMs between the slices where the slice kernel does not form the
+  // sums; with T = fp32 and an inner TC type their operands are read from the
+  // mirror, else from l / u
+  const bool ext = !x.ops;
   const bool from_copy = (T == REMIFA_R_32F) && I != REMIFA_FP32;
+  if (ext && !from_copy) store_x = true;
   const int64_t ldo_l = from_copy ? ldcp : ldl, ldo_u = from_copy ? ldcp : ldu;
   auto lop = [&](int64_t i, int64_t j) {
     return (const void*)(from_copy ? at(cpy, REMIFA_R_16F, i, j, ldcp) : at(l, T, i, j, ldl));
@@ -145,7 +173,7 @@ int inner(Ctx& x, bool rl, int T, int64_t m, int64_t n, int64_t nb, void* l, int
     }
     half_t* const cps = cpy ? (half_t*)at(cpy, REMIFA_R_16F, so, so, ldcp) : nullptr;
     void* const as = at(a, W, so, so, lda);
-    RF_CHECK(slice_launch(x.h, T, W, I, rl, (int)x.ib, x.pw, m, nb, so, sw, so + sw >= n,
+    RF_CHECK(slice_launch(x.h, T, W, I, rl, (int)x.ib, x.pw, m, std::min(nb, m), so, sw, so + sw >= n,
                           at(l, T, so, so, ldl), ldl, at(u, T, so, so, ldu), ldu, store_x, cps,
                           ldcp, x.ops, as, lda, (void*)cps == as ? nullptr : cps, ldcp, col + so,
                           x.pend));
@@ -269,13 +297,9 @@ int side_stream(remifa_handle_t h) {
   return 0;
 }
 
-// fp16 storage factored in fp32 buffers of one block column and block row
-bool buffered_layout(int algo, const remifa_lu_config_t& c) {
-  return algo == REMIFA_LL && c.W == REMIFA_R_16F && c.IP == REMIFA_R_32F;
-}
-
+// sums: bytes of the slices' operand copies
 size_t lu_workspace_bytes(int algo, const remifa_lu_config_t& c, int64_t m, int64_t n, int64_t nb,
-                          bool have_cpy) {
+                          bool have_cpy, size_t sums) {
   size_t b = (2 * slice_slot_bytes() + 255) & ~(size_t)255;  // the slices' tile slots
   if (algo == REMIFA_LL && c.O == REMIFA_BF16_TC32 && c.W == REMIFA_R_16F &&
       c.IP == REMIFA_R_32F)
@@ -301,8 +325,12 @@ size_t lu_workspace_bytes(int algo, const remifa_lu_config_t& c, int64_t m, int6
     b += ((size_t)nb * m * 4 + 255) & ~(size_t)255;
     b += gemm_reserve(m, nb);
   }
-  const int T = buffered_layout(algo, c) ? REMIFA_R_32F : c.W;
-  return b + main_reserve(c, T, m, nb);
+  return b + main_reserve(m, nb, sums);
+}
+
+size_t lu_workspace_bytes(int algo, const remifa_lu_config_t& c, int64_t m, int64_t n, int64_t nb,
+                          bool have_cpy) {
+  return lu_workspace_bytes(algo, c, m, n, nb, have_cpy, slice_sum_bytes(algo, c, m, nb));
 }
 
 int lu_nopiv_impl(remifa_handle_t h, int algo, const remifa_lu_config_t* cfg, int64_t m, int64_t n,
@@ -327,7 +355,13 @@ int lu_nopiv_impl(remifa_handle_t h, int algo, const remifa_lu_config_t* cfg, in
     return 0;
   }
   const bool need_cpy = W == REMIFA_R_32F && (c.I != REMIFA_FP32 || c.O != REMIFA_FP32);
-  const size_t ws = lu_workspace_bytes(algo, c, m, n, nb, d_cpy != nullptr);
+  // (a caller's workspace without room for the operand copies does without)
+  size_t sums = slice_sum_bytes(algo, c, m, nb);
+  size_t ws = lu_workspace_bytes(algo, c, m, n, nb, d_cpy != nullptr, sums);
+  if (h->ws_user && ws > h->ws_bytes) {
+    sums = 0;
+    ws = lu_workspace_bytes(algo, c, m, n, nb, d_cpy != nullptr, sums);
+  }
   RF_CHECK(ensure_workspace(h, ws));
   Arena ar{(char*)h->ws};
   // slice width: a multiple of ib, at most 64 (handle knob, default 64)
@@ -384,12 +418,12 @@ int lu_nopiv_impl(remifa_handle_t h, int algo, const remifa_lu_config_t* cfg, in
     f8.su = (uint8_t*)ar.take((size_t)n * f8.lds8);
   }
   h->ws_used = ar.off;
-  x.ops = (char*)h->ws + ar.off;
+  if (sums) x.ops = (char*)h->ws + ar.off;
   // split-K regions: [ar.off, +R) for the handle's stream (shared with the
   // slices' operand copies), [ar.off + R, +R) for the side stream (the
   // arena's end is lowered while they run)
   const size_t ws_bytes0 = h->ws_bytes;
-  const size_t side_lo = ar.off + main_reserve(c, buffered ? REMIFA_R_32F : W, m, nb);
+  const size_t side_lo = ar.off + main_reserve(m, nb, sums);
   const size_t side_hi = side_lo + gemm_reserve(m, nb);
   if (la_layout || la_inplace) h->ws_bytes = side_lo;
   const int64_t nc = (n - 1) / nb + 1;

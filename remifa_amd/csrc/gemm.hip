@@ -641,10 +641,11 @@ int gemm_dual_launch(remifa_handle_t h, int ctype, int in_t, int64_t m0, int64_t
 }
 
 // The two slice updates of an inner LL factorization whose sums the slice
-// kernel does not form: fp16 sums in one launch; bf16 operands (rounded from
-// the fp16 mirror of fp32 buffers) in one launch when they take the narrow
-// tiles without split-K (C0 -= A0 B0 with N0 <= 32 per tile column, C1 -= A1
-// B1 with M1 <= 64); otherwise two gemm_launch calls.
+// kernel does not form (fp16 sums; bf16 operands rounded from the fp16 mirror
+// of fp32 buffers; outer blocks too wide for its operand copies): fp16 sums in
+// one launch; the others in one launch when they take the narrow tiles without
+// split-K (C0 -= A0 B0 with N0 <= 32 per tile column, C1 -= A1 B1 with M1 <=
+// 64); otherwise two gemm_launch calls.
 int gemm_pair_launch(remifa_handle_t h, int ctype, int in_t, int out_t, int64_t m0, int64_t n0,
                      int64_t k, const void* a0, int64_t lda0, const void* b0, int64_t ldb0,
                      void* c0, int64_t ldc0, int64_t m1, int64_t n1, const void* a1, int64_t lda1,
@@ -660,17 +661,21 @@ int gemm_pair_launch(remifa_handle_t h, int ctype, int in_t, int out_t, int64_t 
     timer_end(h);
     return st;
   }
-  const bool bf = ctype == REMIFA_BF16_TC32 && in_t == REMIFA_R_16F && out_t == REMIFA_R_32F;
+  int opk = -1;
+  if (ctype == REMIFA_FP32 && in_t == REMIFA_R_32F) opk = OPK_F32;
+  if (ctype == REMIFA_TC32 && in_t == REMIFA_R_16F) opk = OPK_F16;
+  if (ctype == REMIFA_BF16_TC32 && in_t == REMIFA_R_16F) opk = OPK_BF16;
+  const int chunk = opk == OPK_F32 ? 4 : 8;
   auto vec_ok = [&](const void* a, int64_t lda, const void* b, int64_t ldb, int64_t m) {
-    return ((uintptr_t)a % 16 == 0) && ((uintptr_t)b % 16 == 0) && (lda % 8 == 0) &&
-           (ldb % 8 == 0) && (m % 8 == 0) && (k % 8 == 0);
+    return ((uintptr_t)a % 16 == 0) && ((uintptr_t)b % 16 == 0) && (lda % chunk == 0) &&
+           (ldb % chunk == 0) && (m % chunk == 0) && (k % chunk == 0);
   };
   // the rule table / overrides must pick the narrow tiles without split-K
   auto rule = [&](int64_t m, int64_t n, int& tile, int& split) {
-    tile = choose_tile(OPK_BF16, m, n);
+    tile = choose_tile(opk, m, n);
     split = 0;
     for (const auto& r : h->gemm_rules)
-      if ((r[0] < 0 || r[0] == OPK_BF16) && m >= r[1] && m <= r[2] && n >= r[3] && n <= r[4]) {
+      if ((r[0] < 0 || r[0] == opk) && m >= r[1] && m <= r[2] && n >= r[3] && n <= r[4]) {
         tile = (int)r[5];
         split = (int)r[6];
         break;
@@ -680,9 +685,9 @@ int gemm_pair_launch(remifa_handle_t h, int ctype, int in_t, int out_t, int64_t 
   rule(m0, n0, t0, s0);
   rule(m1, n1, t1, s1);
   const bool v0 = vec_ok(a0, lda0, b0, ldb0, m0), v1 = vec_ok(a1, lda1, b1, ldb1, m1);
-  const bool pair = bf && k > 0 && m0 > 0 && n0 > 0 && m1 > 0 && n1 > 0 && t0 == T256x32 &&
+  const bool pair = opk >= 0 && k > 0 && m0 > 0 && n0 > 0 && m1 > 0 && n1 > 0 && t0 == T256x32 &&
                     t1 == T32x256 && s0 <= 1 && s1 <= 1 && h->split_k <= 0 && h->gemm_tile < 0 &&
-                    v0 == v1;
+                    v0 == v1 && (out_t == REMIFA_R_32F || (out_t == REMIFA_R_16F && opk != OPK_F32));
   if (!pair) {
     RF_CHECK(gemm_launch(h, ctype, in_t, out_t, m0, n0, k, -1.0f, a0, lda0, b0, ldb0, 1.0f, c0,
                          ldc0));
@@ -699,8 +704,18 @@ int gemm_pair_launch(remifa_handle_t h, int ctype, int in_t, int out_t, int64_t 
   };
   GemmArgs g0 = args(m0, n0, a0, lda0, b0, ldb0, c0, ldc0);
   GemmArgs g1 = args(m1, n1, a1, lda1, b1, ldb1, c1, ldc1);
-  timer_begin(h, KC_GEMM, 2.0 * (double)k * (m0 * n0 + m1 * n1), (OPK_BF16 << 8) | 8);
-  const int st = launch_pair<OPK_BF16, float>(h, g0, g1, v0);
+  timer_begin(h, KC_GEMM, 2.0 * (double)k * (m0 * n0 + m1 * n1),
+              (opk << 8) | ((out_t == REMIFA_R_16F) << 4) | 8);
+  const bool f32 = out_t == REMIFA_R_32F;
+  int st;
+  if (opk == OPK_F32)  // (fp32 buffers only)
+    st = launch_pair<OPK_F32, float>(h, g0, g1, v0);
+  else if (opk == OPK_F16)
+    st = f32 ? launch_pair<OPK_F16, float>(h, g0, g1, v0)
+             : launch_pair<OPK_F16, half_t>(h, g0, g1, v0);
+  else
+    st = f32 ? launch_pair<OPK_BF16, float>(h, g0, g1, v0)
+             : launch_pair<OPK_BF16, half_t>(h, g0, g1, v0);
   timer_end(h);
   return st;
 }

@@ -74,7 +74,7 @@ size_t slice_op_bytes(int T, int I, int64_t m, int64_t nb) {
   return 2 * al256((size_t)(m + SW) * op_ld(nb) * op_size(T, I));
 }
 
-// true if the slice kernel subtracts the earlier slices' products itself;
+// true if the slice kernel can subtract the earlier slices' products itself;
 // else the driver runs the update GEMMs (fp16-accumulated sums; bf16 operands
 // rounded from the fp16 mirror of fp32 buffers)
 bool slice_updates(int T, int I) {
@@ -82,7 +82,8 @@ bool slice_updates(int T, int I) {
 }
 
 // One slice at offset so of the outer block (m rows below and including its
-// first row): l, u, cp point at the slice's diagonal tile.
+// first row): l, u, cp point at the slice's diagonal tile. nb: width of the
+// outer block's operand copies ops (null: the driver runs the update GEMMs).
 //
 // Measured (MI355X): a slice takes 22 us at n = 5001 (fp16 panels, ib = 8, nb
 // = 256) where the tile kernel (30), the vector kernel (22) and the update
@@ -100,16 +101,18 @@ int slice_launch(remifa_handle_t h, int T, int W, int I, bool rl, int ib, int pw
     return REMIFA_ERR_UNSUPPORTED;
   SliceArgs g{};
   g.cm = cm, g.sw = sw, g.so = (int)so, g.chunk = pw;
-  g.pre = so > 0 && slice_updates(T, I);
+  g.pre = so > 0 && ops;
   g.l = l, g.ldl = ldl, g.u = u, g.ldu = ldu, g.store_x = store_x;
   g.cp = cp, g.ldcp = ldcp;
   const int64_t es16 = 16 / (int64_t)dtype_size(T);
   g.vec = (!store_x || ((uintptr_t)u % 16 == 0 && ldu % es16 == 0)) &&
           (!cp || ((uintptr_t)cp % 16 == 0 && ldcp % 8 == 0));
   g.ldop = op_ld(nb);
-  g.lop = ops;
-  g.uop = (char*)ops + al256((size_t)(m + SW) * g.ldop * op_size(T, I));
-  g.write_op = !last && slice_updates(T, I);
+  if (ops) {
+    g.lop = ops;
+    g.uop = (char*)ops + al256((size_t)(m + SW) * g.ldop * op_size(T, I));
+  }
+  g.write_op = !last && ops;
   const int vpu = mode == SM_F32 ? 32 : 64;
   g.nul = (int)ceil_div(cm - sw, vpu);
   g.nunits = 2 * g.nul;
