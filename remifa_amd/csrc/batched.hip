@@ -2,9 +2,9 @@
 // up to 512), fp32 storage with matrix-core updates (TC32: fp16 operands,
 // fp32 accumulation; BF16_TC32: bf16 operands).
 //
-// One persistent launch: a fixed grid of 8-wavefront workgroups takes
-// matrices from an atomic queue (callers order the batch largest first, so
-// the queue is a longest-processing-time schedule). A workgroup factors its
+// One persistent launch: a grid of as many workgroups as the chip holds (or
+// as there are matrices) takes matrices from an atomic queue (callers order
+// the batch largest first, so the queue is a longest-processing-time schedule). A workgroup factors its
 // matrix right-looking with 32-wide panels, which is the reference's RL
 // driver with nb = ib = 32 (src/lu_nopiv.hxx:53-208): per panel
 //  1. the 32 pivots of the panel: lane i keeps row i of the panel in
@@ -15,20 +15,31 @@
 //  2. the block row U12 = L11^-1 A12, one lane per column;
 //  3. the Schur update A22 -= L21 U12 on the matrix cores from fp16 (bf16)
 //     copies of L21 and U12 staged in LDS, products summed from zero and
-//     subtracted once (the update GEMMs of gemm.hip do the same); two
+//     subtracted once (the update GEMMs of gemm.hip do the same); two or four
 //     32 x 32 tiles of C per wavefront in flight together.
 // The matrix stays in HBM; every element of the trailing matrix is read and
-// written once per panel, which is what bounds orders above 256 (about 7 TB/s
-// over the chip); the pivots and the two triangular steps (25 us per panel of
-// order 500, against 24 us of update) run under another workgroup's update.
-// Measured (MI355X), 2000 matrices of order 257 to 512: 4117 us with one
-// workgroup per CU (80 KB of operands, whole columns read entry by entry in 2.),
-// 3360 with two; 129 to 256: 1139 -> 605 us (four workgroups); 65 to 128: 274 ->
-// 170 us (eight).
+// written once per panel, which is what bounds large batches of orders above
+// 256 (about 7 TB/s over the chip); the pivots and the two triangular steps (25
+// us per panel of order 500, against 24 us of update) run under another
+// workgroup's update.
+//
+// Two instantiations. MANY: 128 registers per lane, so that four wavefronts
+// share a SIMD and hide each other's latencies, two tiles of C in flight. The
+// other: one wavefront per SIMD with all its registers (none spilled) and four
+// tiles in flight, for batches whose time is that of a matrix or two per
+// workgroup, and for the smallest orders, whose panels are all latency. Measured
+// (MI355X, us, orders 33 to 64 / 65 to 128 / 129 to 256 / 257 to 512), MANY against
+// the other: 32 matrices 49 / 106 / 257 / 675 and 39 / 82 / 188 / 628; 600 matrices
+// 54 / 122 / 311 / 1240 and 43 / 103 / 351 / 1141; 1500 matrices 79 / 152 / 491 /
+// 2527 and 76 / 188 / 772 / 2619; 4000 matrices 148 / 324 / 1167 / 6681 and 139 /
+// 468 / 2037 / 6931.
 //
 // The batched solve runs one workgroup per matrix: x in LDS, 32-row blocks,
 // the 32x32 diagonal block substitution inside one wavefront, the rest of
 // each block column as a matrix-vector update by all lanes.
+#include <algorithm>
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace remifa {
@@ -70,12 +81,11 @@ __device__ __forceinline__ uint16_t op_bits(float v) {
 
 // BM: largest order taken (a size bucket), BT: threads (BT >= BM: one lane
 // per row of a panel and per column of a block row)
-template <bool BF, int BM, int BT>
-__global__ void __launch_bounds__(BT, 4) batched_lu_kernel(int count, const int* __restrict__ d_n,
-                                                        const int* __restrict__ d_ld,
-                                                        float* const* __restrict__ d_ptrs,
-                                                        int* __restrict__ d_info,
-                                                        int* __restrict__ queue) {
+template <bool BF, int BM, int BT, bool MANY>
+__global__ void __launch_bounds__(BT, MANY ? 4 : 1)
+    batched_lu_kernel(int count, const int* __restrict__ d_n, const int* __restrict__ d_ld,
+                      float* const* __restrict__ d_ptrs, int* __restrict__ d_info,
+                      int* __restrict__ queue) {
   static_assert(BT >= BM && BT >= 64 && BT % 64 == 0, "one lane per row");
   __shared__ BatchLds<BM> S;
   const int t = threadIdx.x;
@@ -213,7 +223,7 @@ __global__ void __launch_bounds__(BT, 4) batched_lu_kernel(int count, const int*
       // ---- 3. A22 -= L21 U12 on the matrix cores, 32 x 32 tiles, two per
       // wavefront at a time (their C entries read in one round trip)
       const int nt = mr32 / 32;
-      constexpr int TQ = 2;
+      constexpr int TQ = MANY ? 2 : 4;
       for (int tile0 = wave; tile0 < nt * nt; tile0 += TQ * (BT / 64)) {
         f16v acc[TQ];
         float cv[TQ][16];
@@ -404,7 +414,8 @@ extern "C" int remifa_lu_nopiv_batched(remifa_handle_t h, int ctype, int64_t cou
   zero_queue_kernel<<<1, 64, 0, h->stream>>>(queue);
   // the size bucket of max_n picks the kernel (LDS for orders up to the
   // bucket's bound) and, from the handle's tuning table, its threads and
-  // persistent workgroups per CU
+  // persistent workgroups per CU; count the instantiation (where the two take
+  // the same time, see above) and at most as many workgroups as matrices
   int bm = 512;
   for (int b : {64, 128, 256})
     if (max_n <= b) {
@@ -413,17 +424,29 @@ extern "C" int remifa_lu_nopiv_batched(remifa_handle_t h, int ctype, int64_t cou
     }
   int bt = 0, per_cu = 0;
   batched_shape(h, bm, &bt, &per_cu);
-  const int grid = per_cu * h->num_cu;
+  const bool many = bm > 64 && count > (bm == 128 ? 4 : (bm == 256 ? 2 : 3)) * (int64_t)h->num_cu;
+  if (!many) per_cu = std::min(per_cu, std::max(1, 256 / bt));  // one wavefront per SIMD
+  const int grid = (int)std::min<int64_t>((int64_t)per_cu * h->num_cu, count);
   timer_begin(h, KC_OTHER, 0.0, 1);
   int st = 0;
-#define RF_BATCHED(BM, BT)                                                                       \
-  if (bm == BM && bt == BT) {                                                                    \
-    if (ctype == REMIFA_TC32)                                                                    \
-      batched_lu_kernel<false, BM, BT>                                                           \
-          <<<grid, BT, 0, h->stream>>>((int)count, d_n, d_ld, d_ptrs, d_info, queue);            \
-    else                                                                                         \
-      batched_lu_kernel<true, BM, BT>                                                            \
-          <<<grid, BT, 0, h->stream>>>((int)count, d_n, d_ld, d_ptrs, d_info, queue);            \
+  auto launch = [&](auto bf, auto bmc, auto btc) {
+    constexpr bool BF = decltype(bf)::value;
+    constexpr int M = decltype(bmc)::value, T = decltype(btc)::value;
+    if (M > 64 && many)
+      batched_lu_kernel<BF, M, T, (M > 64)>
+          <<<grid, T, 0, h->stream>>>((int)count, d_n, d_ld, d_ptrs, d_info, queue);
+    else
+      batched_lu_kernel<BF, M, T, false>
+          <<<grid, T, 0, h->stream>>>((int)count, d_n, d_ld, d_ptrs, d_info, queue);
+  };
+#define RF_BATCHED(BM, BT)                              \
+  if (bm == BM && bt == BT) {                           \
+    using M = std::integral_constant<int, BM>;          \
+    using T = std::integral_constant<int, BT>;          \
+    if (ctype == REMIFA_TC32)                           \
+      launch(std::false_type{}, M{}, T{});              \
+    else                                                \
+      launch(std::true_type{}, M{}, T{});               \
   } else
   RF_BATCHED(64, 64)
   RF_BATCHED(64, 128)
@@ -447,7 +470,7 @@ extern "C" int remifa_lu_nopiv_batched(remifa_handle_t h, int ctype, int64_t cou
 // to bm: the handle's table (remifa_set_batched_tuning) or the defaults.
 void remifa::batched_shape(remifa_handle_t h, int bm, int* bt, int* per_cu) {
   *bt = bm;
-  *per_cu = bm <= 128 ? 8 : (bm <= 256 ? 4 : 2);
+  *per_cu = bm == 128 ? 8 : (bm <= 256 ? 4 : 2);
   for (const auto& r : h->batched_rules)
     if (r[0] == bm) {
       *bt = r[1];

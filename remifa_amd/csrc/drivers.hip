@@ -12,8 +12,8 @@
 // earlier slices of the outer block (LL: one sum; RL: slice by slice, as the
 // rank-pw updates after each slice would) and does the reference's ib loop.
 // fp16-accumulated sums, bf16 ones of fp32 buffers and those of wide outer
-// blocks come from update GEMMs between the slices instead. pw = ib reproduces the reference's
-// structure of one panel per ib columns.
+// blocks come from update GEMMs between the slices instead. pw = ib reproduces
+// the reference's structure of one panel per ib columns.
 //
 // Differences from the reference, all deliberate:
 //  * no allocation inside the loop: one workspace arena per call (slice
