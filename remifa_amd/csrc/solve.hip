@@ -756,7 +756,7 @@ __global__ void __launch_bounds__(256) resid_t_partial_kernel(int64_t n,
 }
 
 // Two to 16 GR right-hand sides: A X (A^T X) on the FP64 matrix cores
-// (16x16x4, A widened in registers), part[chunk][n][16 GR]. A wavefront owns
+// (16x16x4, A widened in registers), part[chunk][n][nrhs]. A wavefront owns
 // 64 entries of the result (rows of A, or columns for A^T), a workgroup 256,
 // over jc columns (rows) of A. Plain: a lane reads four consecutive rows of a
 // column, 16 lanes 256 bytes of it, and component e of the read belongs to
@@ -846,7 +846,8 @@ __global__ void __launch_bounds__(256) resid_mm_kernel(int64_t n, int nrhs,
       if (row < n) {
 #pragma unroll
         for (int g = 0; g < GR; ++g)
-          part[((int64_t)blockIdx.y * n + row) * (16 * GR) + 16 * g + l16] = acc[i][g][j];
+          if (16 * g + l16 < nrhs)
+            part[((int64_t)blockIdx.y * n + row) * nrhs + 16 * g + l16] = acc[i][g][j];
       }
     }
 }
@@ -870,11 +871,11 @@ __device__ __forceinline__ void block_absmax(double v, double* out) {
   }
 }
 
-// r = b - the partials, chunk by chunk (chunk order: deterministic). KW: the
-// partials' right-hand sides per entry (a workgroup takes 256 / KW entries of
-// 16 right-hand sides), or 1: one right-hand side. With w: the fp32 copy the
-// correction solve takes, and max |r| per column, instead of r.
-template <int KW>
+// r = b - the partials, chunk by chunk (chunk order: deterministic). ONE: one
+// right-hand side, else nrhs per entry (a workgroup takes 16 entries of 16
+// right-hand sides). With w: the fp32 copy the correction solve takes, and max
+// |r| per column, instead of r.
+template <bool ONE>
 __global__ void __launch_bounds__(256) resid_reduce_kernel(int64_t n, int nrhs, int nchunk,
                                                            const double* __restrict__ part,
                                                            const double* __restrict__ b,
@@ -882,7 +883,7 @@ __global__ void __launch_bounds__(256) resid_reduce_kernel(int64_t n, int nrhs, 
                                                            int64_t ldr, float* __restrict__ w,
                                                            double* __restrict__ rmax) {
   const int t = threadIdx.x;
-  if constexpr (KW == 1) {
+  if constexpr (ONE) {
     const int64_t i = (int64_t)blockIdx.x * 256 + t;
     double v = 0.0;
     if (i < n) {
@@ -904,7 +905,7 @@ __global__ void __launch_bounds__(256) resid_reduce_kernel(int64_t n, int nrhs, 
     if (i < n && k < nrhs) {
       double s = 0.0;
 #pragma unroll 8
-      for (int c = 0; c < nchunk; ++c) s += part[((int64_t)c * n + i) * KW + k];
+      for (int c = 0; c < nchunk; ++c) s += part[((int64_t)c * n + i) * nrhs + k];
       v = b[i + k * ldb] - s;
       if (w)
         w[i + k * n] = (float)v;
@@ -1149,13 +1150,14 @@ int getrs_launch(remifa_handle_t h, int lu_t, int trans, int64_t n, int64_t nrhs
   return st;
 }
 
-// right-hand sides of one residual pass: one, or 16 to 64 on the matrix cores
-// (lean: one at a time, whose partials fit wherever a call was accepted
-// before), and the chunks its sum over A is cut into (enough workgroups to
-// fill the chip, at least 256 long)
+// right-hand sides of one residual pass: one, or up to 16, 32 or 64 on the
+// matrix cores (lean: up to 16, for a caller's workspace: partials of 16
+// columns in chunks of 256 fit the smallest accepted one), and the chunks its
+// sum over A is cut into (enough workgroups to fill the chip, at least 256
+// long)
 static int resid_group(int64_t nrhs, bool lean) {
-  if (nrhs == 1 || lean) return 1;
-  return (nrhs <= RES_RHS ? 1 : (nrhs <= 2 * RES_RHS ? 2 : 4)) * RES_RHS;
+  if (nrhs == 1) return 1;
+  return (nrhs <= RES_RHS || lean ? 1 : (nrhs <= 2 * RES_RHS ? 2 : 4)) * RES_RHS;
 }
 static int64_t resid_chunks(int64_t n, int trans, int kw) {
   if (kw == 1) return trans ? ceil_div(n, RES_T1) : ceil_div(n, RES_COLS);
@@ -1166,7 +1168,7 @@ static size_t resid_part_bytes(int64_t n, int64_t nrhs, bool lean) {
   const int kw = resid_group(nrhs, lean);
   // the largest of the two layouts
   const int64_t ch = std::max(resid_chunks(n, 0, kw), resid_chunks(n, 1, kw));
-  return sizeof(double) * (size_t)ch * (size_t)kw * (size_t)n;
+  return sizeof(double) * (size_t)ch * (size_t)std::min<int64_t>(kw, nrhs) * (size_t)n;
 }
 
 // R = B - A X (A^T X when trans): to r, or to w (fp32, leading dimension n)
@@ -1196,7 +1198,7 @@ int residual_launch(remifa_handle_t h, int64_t n, int64_t nrhs, const float* a, 
       else
         resid_partial_kernel<<<dim3((unsigned)ceil_div(n, RES_ROWS), nchunk), 256, 0, s>>>(
             n, a, lda, xk, part);
-      resid_reduce_kernel<1><<<(unsigned)ceil_div(n, 256), 256, 0, s>>>(n, 1, nchunk, part, bk,
+      resid_reduce_kernel<true><<<(unsigned)ceil_div(n, 256), 256, 0, s>>>(n, 1, nchunk, part, bk,
                                                                         ldb, rk, ldr, wk, mk);
       continue;
     }
@@ -1207,7 +1209,7 @@ int residual_launch(remifa_handle_t h, int64_t n, int64_t nrhs, const float* a, 
     resid_mm_kernel<GR, true><<<g1, 256, 0, s>>>(n, nr, a, lda, xk, ldx, part, jc, vec);        \
   else                                                                                          \
     resid_mm_kernel<GR, false><<<g1, 256, 0, s>>>(n, nr, a, lda, xk, ldx, part, jc, vec);       \
-  resid_reduce_kernel<16 * GR><<<g2, 256, 0, s>>>(n, nr, nchunk, part, bk, ldb, rk, ldr, wk, mk)
+  resid_reduce_kernel<false><<<g2, 256, 0, s>>>(n, nr, nchunk, part, bk, ldb, rk, ldr, wk, mk)
     if (kw == RES_RHS) {
       RF_RESID(1);
     } else if (kw == 2 * RES_RHS) {
