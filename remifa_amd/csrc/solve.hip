@@ -1151,23 +1151,27 @@ int getrs_launch(remifa_handle_t h, int lu_t, int trans, int64_t n, int64_t nrhs
 }
 
 // right-hand sides of one residual pass: one, or up to 16, 32 or 64 on the
-// matrix cores (lean: up to 16, for a caller's workspace: partials of 16
-// columns in chunks of 256 fit the smallest accepted one), and the chunks its
-// sum over A is cut into (enough workgroups to fill the chip, at least 256
-// long)
+// matrix cores; lean: up to 16 in chunks of 256, for a caller's workspace (the
+// smallest accepted one holds their partials)
 static int resid_group(int64_t nrhs, bool lean) {
   if (nrhs == 1) return 1;
   return (nrhs <= RES_RHS || lean ? 1 : (nrhs <= 2 * RES_RHS ? 2 : 4)) * RES_RHS;
 }
-static int64_t resid_chunks(int64_t n, int trans, int kw) {
+// Chunks that the sum over A is cut into: enough workgroups to fill the chip,
+// two (16 columns four) per CU, each chunk at least one staged piece of 32
+// long. Measured (MI355X, us, 16 columns, two with chunks of 256 against four):
+// n = 130 27 / 12, n = 1000 40 / 13, n = 12000 324 / 215, n = 20000 832 / 560 (eight
+// per CU: n = 12000 182, n = 8000 76 against 66).
+static int64_t resid_chunks(int64_t n, int trans, int kw, bool lean) {
   if (kw == 1) return trans ? ceil_div(n, RES_T1) : ceil_div(n, RES_COLS);
-  return std::min(ceil_div(n, 256), std::max<int64_t>(1, ceil_div(512, ceil_div(n, 256))));
+  const int64_t want = ceil_div(kw == RES_RHS ? 1024 : 512, ceil_div(n, 256));
+  return std::min(ceil_div(n, lean ? 256 : 32), want);
 }
 
 static size_t resid_part_bytes(int64_t n, int64_t nrhs, bool lean) {
   const int kw = resid_group(nrhs, lean);
   // the largest of the two layouts
-  const int64_t ch = std::max(resid_chunks(n, 0, kw), resid_chunks(n, 1, kw));
+  const int64_t ch = std::max(resid_chunks(n, 0, kw, lean), resid_chunks(n, 1, kw, lean));
   return sizeof(double) * (size_t)ch * (size_t)std::min<int64_t>(kw, nrhs) * (size_t)n;
 }
 
@@ -1184,7 +1188,7 @@ int residual_launch(remifa_handle_t h, int64_t n, int64_t nrhs, const float* a, 
   const int vec = (uintptr_t)a % 16 == 0 && lda % 4 == 0;
   for (int64_t k0 = 0; k0 < nrhs; k0 += kw) {
     const int nr = (int)std::min<int64_t>(kw, nrhs - k0);
-    const int nchunk0 = (int)resid_chunks(n, trans, kw);
+    const int nchunk0 = (int)resid_chunks(n, trans, kw, lean);
     const int64_t jc = ceil_div(ceil_div(n, nchunk0), 32) * 32;
     const int nchunk = kw == 1 ? nchunk0 : (int)ceil_div(n, jc);
     const double *xk = x + k0 * ldx, *bk = b + k0 * ldb;
