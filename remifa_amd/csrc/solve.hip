@@ -634,42 +634,50 @@ __global__ void __launch_bounds__(TT) trsm16_kernel(int64_t n, int nrhs, int ngr
     acc = product(tv, xs[q & 1], acc);
   }
   float* const xr = xs[nsteps & 1];
-  bool finite = true;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int rr = 16 * w + 4 * lq + j;
-    const float v = bv[j] - acc[j];
-    xr[(rr % KS) * XP + (rr / KS) * RC + l16] = v;
-    finite &= __builtin_isfinite(v);
+    xr[(rr % KS) * XP + (rr / KS) * RC + l16] = bv[j] - acc[j];
   }
   __syncthreads();
-  f4v y = product(dv, xr, (f4v){0.0f, 0.0f, 0.0f, 0.0f}), yd = y;
-  if (__ballot(!finite) != 0) {
-    // an infinite entry times the diagonal's place, now zero, is NaN: where
-    // an entry is not finite its row takes the product with the diagonal in it
-    const float d0 = inv[((int64_t)bi * NBS + 16 * w + l16) * NBS + 16 * w + l16];
-#pragma unroll
-    for (int s = 0; s < KS; ++s)
-      if (32 * lq + s == 16 * w + l16) dv[s] = d0;
-    yd = product(dv, xr, (f4v){0.0f, 0.0f, 0.0f, 0.0f});
-  }
-  f4v z = {0.0f, 0.0f, 0.0f, 0.0f};
+  f4v y = product(dv, xr, (f4v){0.0f, 0.0f, 0.0f, 0.0f}), z = {0.0f, 0.0f, 0.0f, 0.0f};
   if (fold) {
     float* const xn = xs[(nsteps + 1) & 1];
     stage(tk - 1, xn);
     z = product(mv, xn, z);
+    y -= z;
+  }
+  bool nan = false;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    y[j] = __builtin_fmaf(dd[j], bv[j] - acc[j], y[j]);
+    nan |= y[j] != y[j];
+  }
+  if (__ballot(nan) != 0) {
+    // an infinite entry times the diagonal's place, zero above, is NaN: where
+    // an entry is not finite its row takes the product with the diagonal in it
+    const float* const ib = inv + (int64_t)bi * NBS * NBS;
+    f4v yd = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 16
+    for (int s = 0; s < KS; ++s)
+      yd = __builtin_amdgcn_mfma_f32_16x16x4f32(TRANS ? ib[(32 * lq + s) * NBS + 16 * w + l16]
+                                                      : ib[(16 * w + l16) * NBS + 32 * lq + s],
+                                                xr[s * XP + lane], yd, 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (!__builtin_isfinite(bv[j] - acc[j])) y[j] = yd[j] - z[j];
   }
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const float v = bv[j] - acc[j];
-    y[j] = __builtin_isfinite(v) ? __builtin_fmaf(dd[j], v, y[j] - z[j]) : yd[j] - z[j];
     if (go + j < n && l16 < nr) {
       __hip_atomic_store(&tags[go + j + (int64_t)l16 * n],
                          (1ull << 32) | (unsigned long long)__float_as_uint(y[j]),
                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      b[go + j + l16 * ldb] = y[j];  // the caller's copy
     }
   }
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (go + j < n && l16 < nr) b[go + j + l16 * ldb] = y[j];  // the caller's copy
 }
 
 // clears the sync words (the error flag only if asked: it is kept over the
