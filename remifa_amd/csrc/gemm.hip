@@ -165,12 +165,13 @@ int splitk_reduce_launch(remifa_handle_t h, int out_t, int64_t m, int64_t n, int
 // (the LU's updates: less than a wavefront per SIMD), the serial K chain. A
 // wavefront takes 128 rows (a row pair per lane) and NC columns, a workgroup
 // 4 NC columns of the same rows. The lanes read their rows of A straight from
-// memory through a ring of KU registers, each refilled as soon as it is used,
-// so KU loads are in flight whatever the latency (the other three wavefronts
-// hit the same lines); the columns of B are uniform over a wavefront and come
-// from LDS as 16-byte broadcasts of eight k-values. Measured (MI355X) over
-// the updates of the n = 3000 factorization (nb = 256): 2.0 against 10.1 ms
-// with 64 x 64 tiles, both operands in LDS and scalar fma.
+// memory through a ring of KU registers, each refilled as soon as it is used
+// (the other three wavefronts hit the same lines); the columns of B are uniform
+// over a wavefront and come from LDS as 16-byte broadcasts of eight k-values.
+// Three to four wavefronts per SIMD hide the rest of the latency: a ring of 48
+// took all registers for one. Measured (MI355X, us; 64 x 64 tiles with both
+// operands in LDS and scalar fma / ring of 48 / this one): 5000^2 K = 8 47 / 181 /
+// 45, K = 128 237 / 345 / 112; 1024^2 K = 64 16 / 20 / 9, K = 1500 255 / 135 / 83.
 struct HalfGemm {
   int64_t M, N, K;
   const half_t* A;
@@ -191,7 +192,7 @@ typedef hh2 hh2u __attribute__((aligned(2)));
 template <int NC>
 __global__ void __launch_bounds__(256) gemm_h16_kernel(HalfGemm g0, HalfGemm g1, int nt0,
                                                        half_t alpha, half_t beta) {
-  constexpr int KU = 48;                 // k-values per slab and registers of the ring
+  constexpr int KU = 16;                 // k-values per slab and registers of the ring
   constexpr int NL = 4 * NC * KU / 256;  // elements of B per thread and slab
   __shared__ __attribute__((aligned(16))) half_t Bs[2][4 * NC][KU];
   const bool first = (int)blockIdx.x < nt0;
@@ -257,7 +258,7 @@ __global__ void __launch_bounds__(256) gemm_h16_kernel(HalfGemm g0, HalfGemm g1,
           p += g.lda;
         }
       }
-      if constexpr (REFILL) __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
   if (g.K > 0) {
@@ -276,32 +277,51 @@ __global__ void __launch_bounds__(256) gemm_h16_kernel(HalfGemm g0, HalfGemm g1,
       slab(buf, k0, std::integral_constant<bool, false>{});
       if (more) load_a(k0 + KU);
     } else {
+      // the last k-values, eight at a time
       const half_t(*const bs)[KU] = &Bs[buf][wave * NC];
       const int kn = (int)(g.K - k0);
 #pragma unroll
-      for (int k = 0; k < KU; ++k) {
-        if (k < kn) {
+      for (int kk = 0; kk < KU; kk += 8) {
+        if (kk < kn) {
+          h8 b[NC];
 #pragma unroll
-          for (int c = 0; c < NC; ++c) {
-            const half_t b = bs[c][k];
-            acc[c] = __builtin_elementwise_fma(a[k], (hh2){b, b}, acc[c]);
-          }
+          for (int c = 0; c < NC; ++c) b[c] = *(const h8*)&bs[c][kk];
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            if (kk + j < kn) {
+#pragma unroll
+              for (int c = 0; c < NC; ++c)
+                acc[c] = __builtin_elementwise_fma(a[kk + j], (hh2){b[c][j], b[c][j]}, acc[c]);
+            }
+          __builtin_amdgcn_sched_barrier(0);
         }
       }
     }
     if (more) store_b(buf ^ 1);
   }
+  // (every entry of C is requested before the first is written)
+  const int64_t nb = n0 + wave * NC;
+  half_t* const cb = g.C + row0;
+  hh2 cv[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    const int64_t n = n0 + wave * NC + c;
-    if (n >= g.N) continue;
+    cv[c] = (hh2){(_Float16)0, (_Float16)0};
+    if (beta != (half_t)0) cv[c] = *(const hh2u*)(cb + (nb + c < g.N ? nb + c : g.N - 1) * g.ldc);
+  }
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    hh2 r;
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
-      if (row0 + e >= row) {
-        half_t* const cp = g.C + row0 + e + n * g.ldc;
-        const half_t bc = (beta != (half_t)0) ? beta * *cp : (half_t)0;
-        *cp = __builtin_fmaf16(alpha, acc[c][e], bc);
-      }
+      const half_t bc = (beta != (half_t)0) ? beta * cv[c][e] : (half_t)0;
+      r[e] = __builtin_fmaf16(alpha, acc[c][e], bc);
+    }
+    half_t* const cp = cb + (nb + c) * g.ldc;
+    if (nb + c < g.N) {
+      if (row0 == row)
+        *(hh2u*)cp = r;
+      else if (row0 + 1 == row)
+        cp[1] = r[1];
     }
   }
 }

@@ -65,14 +65,14 @@ def test_wide_blocks_match_oracle(handle, gpu, name, algo, n, nb, pad):
     assert_parity(to_np(d), o, f"{name} {algo} n={n} nb={nb}")
 
 
-@pytest.mark.parametrize("name", ["f16tc", "buftc", "f32tc"])
-def test_workspace_without_operand_copies(gpu, name):
+@pytest.mark.parametrize("name,n,nb", [("f16bf", 8192, 8192), ("f16tc", 16384, 4096),
+                                       ("f32tc", 16384, 4096)])
+def test_workspace_without_operand_copies(gpu, name, n, nb):
     """A caller's workspace that holds everything but the operand copies (the
-    split-K partials are capped at 256 MiB, the copies of one block of 8192
-    take 272) is accepted, and its factors refine to FP64 accuracy."""
+    split-K partials are capped at 256 MiB, the copies take more) is accepted,
+    and its factors refine to FP64 accuracy."""
     import torch
     import remifa_amd as rf
-    n = 8192
     W, _, _, OP = TUPLES[name]
     gen = torch.Generator(device="cuda").manual_seed(7)
     a = (torch.rand((n, n), generator=gen, device=gpu) * 2 - 1).t()
@@ -80,16 +80,16 @@ def test_workspace_without_operand_copies(gpu, name):
     b = rf.colmajor_empty(n, 1, dtype=torch.float64)
     b.copy_(torch.rand((n, 1), generator=gen, device=gpu, dtype=torch.float64))
     size = (256 << 20) + (1 << 17)  # partials; the tile slots
-    size += 2 * 4 * n * n if W and not OP else 0  # block column and block row buffers
-    size += 2 * n * n if not W else 0             # the fp16 copy
+    # the fp16 copy, and the second stream's partials
+    size += 0 if W else 2 * n * n + (256 << 20)
     h = rf.Handle()
     ws = torch.empty(size, dtype=torch.uint8, device=gpu)
     h.set_workspace(ws)
     cfg = _cfg(rf, name, 8)
-    assert rf.lu_workspace_size(h, rf.LL, cfg, n, n, n) > size
+    assert rf.lu_workspace_size(h, rf.LL, cfg, n, n, nb) > size
     lu = rf.colmajor_empty(n, n, dtype=torch.float16 if W else torch.float32)
     lu.copy_(a)
-    assert rf.lu_nopiv(h, lu, n, algo=rf.LL, cfg=cfg) == 0
+    assert rf.lu_nopiv(h, lu, nb, algo=rf.LL, cfg=cfg) == 0
     x = torch.empty_like(b)
     it, be, _ = rf.ir_solve(rf.Handle(), a, lu, b, x, tol=1e-14, maxit=30)
     assert it >= 0 and be <= 1e-14
