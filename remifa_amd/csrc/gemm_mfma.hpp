@@ -429,28 +429,31 @@ __device__ __forceinline__ void gemm_mfma_body(const GemmArgs& g, int bid, int b
   } else {
     // A chunk past the last row reads on into the next column, except in A's
     // last column; a short slab's chunks would leave the K range: that slab is
-    // masked (lda >= CH keeps the last column but one inside A)
+    // masked (lda >= CH keeps the last column but one inside A). No other slab:
+    // the masked loop alone.
     const bool mask_last =
         klen % BK != 0 || (kend == g.K && g.M % CH != 0 && m0 + BM >= g.M);
     const int nfull = !(off32 && g.lda >= CH) ? 0 : (mask_last ? nk - 1 : nk);
-    auto load = [&](int kt) {
-      if (kt < nfull)
-        load_slab(kt, std::integral_constant<bool, true>{});
-      else
-        load_slab(kt, std::integral_constant<bool, false>{});
-    };
-    if (nk > 0) {
+    if (nfull <= 0) {
+      run(std::integral_constant<bool, false>{});
+    } else {
+      auto load = [&](int kt) {
+        if (kt < nfull)
+          load_slab(kt, std::integral_constant<bool, true>{});
+        else
+          load_slab(kt, std::integral_constant<bool, false>{});
+      };
       load(0);
       store_tiles(0, std::integral_constant<bool, true>{});
-    }
-    __syncthreads();
-    for (int kt = 0; kt < nk; ++kt) {
-      const int buf = kt & 1;
-      const bool more = kt + 1 < nk;
-      if (more) load(kt + 1);
-      compute(buf);
-      if (more) store_tiles(buf ^ 1, std::integral_constant<bool, true>{});
       __syncthreads();
+      for (int kt = 0; kt < nk; ++kt) {
+        const int buf = kt & 1;
+        const bool more = kt + 1 < nk;
+        if (more) load(kt + 1);
+        compute(buf);
+        if (more) store_tiles(buf ^ 1, std::integral_constant<bool, true>{});
+        __syncthreads();
+      }
     }
   }
 
