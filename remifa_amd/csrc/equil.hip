@@ -59,38 +59,52 @@ __global__ void fill_u32_kernel(unsigned* p, int64_t n) {
 }
 
 // rmax[i] = max_j |a_ij| (as float bits): four rows per thread, eight
-// columns' loads in flight. Measured (MI355X) at 16384 x 16384: 244 us, 4.4 TB/s
-// (one row per thread: 298 us).
+// columns' loads in flight; the threads along the columns meet in LDS, so that
+// few rows are not one atomic per thread on a few words. A grid has at most
+// 65535 workgroups along the columns: each takes chunks of EQ_COLS that far
+// apart. Measured (MI355X) at 16384 x 16384: 244 us, 4.4 TB/s (one row per
+// thread: 298 us).
 __global__ void __launch_bounds__(256) row_absmax_kernel(int64_t m, int64_t n,
                                                          const float* __restrict__ a, int64_t lda,
                                                          unsigned* __restrict__ rmax) {
+  __shared__ float4 part[256];
   const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-  if (i >= m) return;
-  const int64_t j0 = (int64_t)blockIdx.y * EQ_COLS;
-  const int64_t j1 = std::min<int64_t>(n, j0 + EQ_COLS);
   const int dj = blockDim.y;
   float mx[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  int64_t j = j0 + threadIdx.y;
-  if (i + 4 <= m) {
-    for (; j + 7 * dj < j1; j += 8 * dj) {
-      f4 v[8];
+  for (int64_t j0 = (int64_t)blockIdx.y * EQ_COLS; j0 < n; j0 += (int64_t)gridDim.y * EQ_COLS) {
+    const int64_t j1 = std::min<int64_t>(n, j0 + EQ_COLS);
+    int64_t j = j0 + threadIdx.y;
+    if (i + 4 <= m) {
+      for (; j + 7 * dj < j1; j += 8 * dj) {
+        f4 v[8];
 #pragma unroll
-      for (int c = 0; c < 8; ++c) v[c] = ld4(a + i + (j + c * dj) * lda);
+        for (int c = 0; c < 8; ++c) v[c] = ld4(a + i + (j + c * dj) * lda);
 #pragma unroll
-      for (int c = 0; c < 8; ++c)
+        for (int c = 0; c < 8; ++c)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) mx[r] = fmaxf(mx[r], fabsf(v[c].e[r]));
+          for (int r = 0; r < 4; ++r) mx[r] = fmaxf(mx[r], fabsf(v[c].e[r]));
+      }
+      for (; j < j1; j += dj) {
+        const f4 v = ld4(a + i + j * lda);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) mx[r] = fmaxf(mx[r], fabsf(v.e[r]));
+      }
+    } else if (i < m) {
+      for (; j < j1; j += dj)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          mx[r] = fmaxf(mx[r], fabsf(a[(i + r < m ? i + r : i) + j * lda]));
     }
-    for (; j < j1; j += dj) {
-      const f4 v = ld4(a + i + j * lda);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) mx[r] = fmaxf(mx[r], fabsf(v.e[r]));
+  }
+  if (dj > 1) {  // (uniform)
+    part[threadIdx.y * blockDim.x + threadIdx.x] = make_float4(mx[0], mx[1], mx[2], mx[3]);
+    __syncthreads();
+    if (threadIdx.y > 0) return;
+    for (int y = 1; y < dj; ++y) {
+      const float4 v = part[y * blockDim.x + threadIdx.x];
+      mx[0] = fmaxf(mx[0], v.x), mx[1] = fmaxf(mx[1], v.y);
+      mx[2] = fmaxf(mx[2], v.z), mx[3] = fmaxf(mx[3], v.w);
     }
-  } else {
-    for (; j < j1; j += dj)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        mx[r] = fmaxf(mx[r], fabsf(a[(i + r < m ? i + r : i) + j * lda]));
   }
 #pragma unroll
   for (int r = 0; r < 4; ++r)
@@ -347,8 +361,9 @@ int remifa_geequb(remifa_handle_t h, int64_t m, int64_t n, const float* d_a, int
   hipStream_t s = h->stream;
   fill_u32_kernel<<<(unsigned)ceil_div(m, 256), 256, 0, s>>>(rmax, m);
   const int bx = eq_rows_of_block(m);
-  row_absmax_kernel<<<dim3((unsigned)ceil_div(m, 4 * bx), (unsigned)ceil_div(n, EQ_COLS)),
-                      dim3(bx, 256 / bx), 0, s>>>(m, n, d_a, lda, rmax);
+  const unsigned gy = (unsigned)std::min<int64_t>(ceil_div(n, EQ_COLS), 65535);
+  row_absmax_kernel<<<dim3((unsigned)ceil_div(m, 4 * bx), gy), dim3(bx, 256 / bx), 0, s>>>(
+      m, n, d_a, lda, rmax);
   row_scale_kernel<<<1, 1024, 0, s>>>(m, rmax, d_r, out, dinfo);
   col_absmax_kernel<<<(unsigned)n, 256, 0, s>>>(m, n, d_a, lda, d_r, dinfo, d_c);
   col_scale_kernel<<<1, 1024, 0, s>>>(m, n, d_c, out, dinfo);
