@@ -165,12 +165,15 @@ _GEMM_TILE = {0: (256, 32, 4, 1), 1: (32, 256, 1, 4), 2: (256, 64, 4, 1), 3: (64
 
 
 def gemm_variant_name(v: int) -> str:
-    """Template instantiation of gemm_mfma_kernel for a GEMM variant code."""
+    """Kernel (and its template instantiation) for a GEMM variant code."""
     opk, out16, tile = v >> 8, (v >> 4) & 15, v & 15
     bm, bn, wm, wn = _GEMM_TILE.get(tile, (0, 0, 0, 0))
+    if opk == 3 and tile == 15:
+        return (f"splitk_reduce_kernel<{'_Float16' if out16 else 'float'}> "
+                f"(split-K partial sums, scaled e4m3 operands)")
     if opk == 3:
-        return (f"gemm_fp8_kernel<{'_Float16' if out16 else 'float'}> "
-                f"(scaled e4m3 operands, 128x128 tile)")
+        return (f"gemm_fp8{'_big' if tile == 4 else ''}_kernel<{'_Float16' if out16 else 'float'}>"
+                f" (scaled e4m3 operands, {bm}x{bn} tile{', LDS-DMA slabs' if tile == 4 else ''})")
     if tile == 15:
         return f"splitk_reduce_kernel<{'_Float16' if out16 else 'float'}> (split-K partial sums)"
     if tile == 8:
