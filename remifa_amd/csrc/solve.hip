@@ -187,17 +187,13 @@ __global__ void __launch_bounds__(TT) trsm_kernel(int64_t n, const LT* __restric
                                                   int* __restrict__ ticket, int* __restrict__ err,
                                                   unsigned long long* __restrict__ tags,
                                                   int nblk) {
-  constexpr int NR = 1, nrhs = 1;
-  constexpr int64_t ldb = 0;
   constexpr int CH = 2;  // solution blocks staged in LDS at a time
-  constexpr int NP = 1;
   // Xs and Red share their LDS with the near block of T, which is only read
   // before the first solution block is staged (a barrier between)
-  constexpr int XS_N = CH * NBS * NR, RED_N = 4 * NBS * NP, TS_N = NBS * NBS;
-  constexpr int U_N = XS_N + RED_N > TS_N ? XS_N + RED_N : TS_N;
-  __shared__ __attribute__((aligned(16))) float ush[U_N];
-  float(*const Xs)[NR] = reinterpret_cast<float(*)[NR]>(ush);
-  float(*const Red)[NBS][NP] = reinterpret_cast<float(*)[NBS][NP]>(ush + XS_N);
+  static_assert(CH * NBS + 4 * NBS <= NBS * NBS, "shared with the near block");
+  __shared__ __attribute__((aligned(16))) float ush[NBS * NBS];
+  float* const Xs = ush;
+  float(*const Red)[NBS] = reinterpret_cast<float(*)[NBS]>(ush + CH * NBS);
   float(*const Ts)[NBS] = reinterpret_cast<float(*)[NBS]>(ush);
   __shared__ int s_ticket;
   const int t = threadIdx.x;
@@ -209,71 +205,59 @@ __global__ void __launch_bounds__(TT) trsm_kernel(int64_t n, const LT* __restric
   const int bi = LOWER ? tk : nblk - 1 - tk;
   const int64_t gr = (int64_t)bi * NBS + row;
 
-  // this lane's entries of the inverted diagonal block (transposed for the
-  // transposed triangles: (T_ii)^-1 = ((D_ii)^-1)^T)
-  float dv[QC];
-  {
-    const float* ib = inv + (int64_t)bi * NBS * NBS;
-#pragma unroll
-    for (int c = 0; c < QC; ++c) {
-      const int col = cq * QC + c;
-      dv[c] = TRANS ? ib[col * NBS + row] : ib[row * NBS + col];
-    }
-  }
-  float acc[NR];
-#pragma unroll
-  for (int k = 0; k < NR; ++k) acc[k] = 0.0f;
-
   // The last dependency (block tk-1 in dependency order, the "near" block)
   // is folded into the diagonal block's inverse ahead of time, M =
   // (T_ii)^-1 T_i,near, so that once X_near is published only X_i = C - M
   // X_near remains (one product and one reduction), with C = (T_ii)^-1 (B_i
   // - sum over the other blocks) formed while waiting.
-  constexpr bool FOLD = true;
-  const bool fold = FOLD && tk >= kFoldFrom;
+  const bool fold = tk >= kFoldFrom;
   const int nsteps = fold ? tk - 1 : tk;  // blocks summed before the wait for the near one
   // rows of the stored factors start on 16 bytes (16-byte vector reads of
   // the transposed triangle's rows)
   const bool vec_rows =
       TRANS && ((uintptr_t)lu % 16 == 0) && (ld % (16 / (int64_t)sizeof(LT)) == 0);
   const int64_t grc = gr < n ? gr : n - 1;  // in-bounds row for the loads
-  // one right-hand side: this lane's entry of b (lanes cq = 0), loaded now
-  // so that no memory round trip follows the last dependency wait (only
-  // this workgroup writes these rows of b). With 16 right-hand sides the
-  // extra registers would spill; those are loaded after the waits.
-  const float bpf = NR == 1 ? b[grc] : 0.0f;
-  float mv[QC];
-  // (T_ii)^-1 in LDS (rows padded against bank conflicts) for M; with one
-  // right-hand side it stays there for the diagonal product, which frees
-  // the lane's registers for the loop
+  // (T_ii)^-1 in LDS (rows padded against bank conflicts; transposed for the
+  // transposed triangles: (T_ii)^-1 = ((D_ii)^-1)^T), for M and the diagonal
+  // product
   __shared__ float Ds[NBS][NBS + 1];
-  if constexpr (FOLD) {
-    if (NR == 1 || fold) {
+  {
+    float dv[QC];
+    const float* ib = inv + (int64_t)bi * NBS * NBS;
 #pragma unroll
-      for (int c = 0; c < QC; ++c) Ds[row][cq * QC + c] = dv[c];
+    for (int c = 0; c < QC; ++c) {
+      const int col = cq * QC + c;
+      dv[c] = TRANS ? ib[col * NBS + row] : ib[row * NBS + col];
     }
-    if (fold) {
-      // M: this lane's row and column quarter, from (T_ii)^-1 and T_i,near
-      // in LDS
-      const int bjn = LOWER ? tk - 1 : nblk - 1 - (tk - 1);
-      const int64_t c0 = (int64_t)bjn * NBS + cq * QC;
 #pragma unroll
-      for (int c = 0; c < QC; ++c) {
-        const int64_t C = c0 + c < n ? c0 + c : n - 1;
-        const float v = tel<LT, TRANS>(lu, ld, grc, C);
-        Ts[row][cq * QC + c] = (gr < n && c0 + c < n) ? v : 0.0f;
-      }
-      __syncthreads();
+    for (int c = 0; c < QC; ++c) Ds[row][cq * QC + c] = dv[c];
+  }
+  // this lane's entry of b (lanes cq = 0), loaded now so that no memory round
+  // trip follows the last dependency wait (only this workgroup writes these
+  // rows of b)
+  const float bv = b[grc];
+  float mv[QC];
+  if (fold) {
+    // M: this lane's row and column quarter, from (T_ii)^-1 and T_i,near in
+    // LDS
+    const int bjn = LOWER ? tk - 1 : nblk - 1 - (tk - 1);
+    const int64_t c0 = (int64_t)bjn * NBS + cq * QC;
 #pragma unroll
-      for (int c = 0; c < QC; ++c) mv[c] = 0.0f;
+    for (int c = 0; c < QC; ++c) {
+      const int64_t C = c0 + c < n ? c0 + c : n - 1;
+      const float v = tel<LT, TRANS>(lu, ld, grc, C);
+      Ts[row][cq * QC + c] = (gr < n && c0 + c < n) ? v : 0.0f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < QC; ++c) mv[c] = 0.0f;
 #pragma unroll 2
-      for (int k = 0; k < NBS; ++k) {
-        const float d = Ds[row][k];
+    for (int k = 0; k < NBS; ++k) {
+      const float d = Ds[row][k];
 #pragma unroll
-        for (int c = 0; c < QC; ++c) mv[c] = __builtin_fmaf(d, Ts[k][cq * QC + c], mv[c]);
-      }
-      __syncthreads();  // (Ts is Xs and Red from here on)
+      for (int c = 0; c < QC; ++c) mv[c] = __builtin_fmaf(d, Ts[k][cq * QC + c], mv[c]);
     }
+    __syncthreads();  // (Ts is Xs and Red from here on)
   }
   // the solution blocks s0 .. s0 + cnt - 1 (dependency order) into Xs:
   // agent-scope atomic loads of the tagged words, each wavefront retrying
@@ -283,20 +267,18 @@ __global__ void __launch_bounds__(TT) trsm_kernel(int64_t n, const LT* __restric
   auto stage_blocks = [&](int s0, int cnt) {
     for (long long tries = 0;; ++tries) {
       int bad = 0;
-      for (int e = t; e < cnt * NBS * NR; e += TT) {
-        const int rr = e % (cnt * NBS), k = e / (cnt * NBS);
-        const int q = rr / NBS, c = rr % NBS;
+      for (int e = t; e < cnt * NBS; e += TT) {
+        const int q = e / NBS, c = e % NBS;
         const int bj = LOWER ? s0 + q : nblk - 1 - (s0 + q);
         const int64_t C = (int64_t)bj * NBS + c;
         float v = 0.0f;
-        if (C < n && k < nrhs) {
-          const unsigned long long w = __hip_atomic_load(&tags[C + (int64_t)k * n],
-                                                         __ATOMIC_RELAXED,
-                                                         __HIP_MEMORY_SCOPE_AGENT);
+        if (C < n) {
+          const unsigned long long w =
+              __hip_atomic_load(&tags[C], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           bad |= (unsigned)(w >> 32) != 1u;
           v = __uint_as_float((unsigned)w);
         }
-        Xs[rr][k] = v;
+        Xs[e] = v;
       }
       if (__ballot(bad) == 0) break;
       if (tries > kSpinLimit ||
@@ -311,6 +293,7 @@ __global__ void __launch_bounds__(TT) trsm_kernel(int64_t n, const LT* __restric
     }
     __syncthreads();
   };
+  float acc = 0.0f;
   for (int s0 = 0; s0 < nsteps; s0 += CH) {
     const int cnt = nsteps - s0 < CH ? nsteps - s0 : CH;
     // this lane's entries of the chunk's blocks of T: issued before the wait
@@ -356,87 +339,43 @@ __global__ void __launch_bounds__(TT) trsm_kernel(int64_t n, const LT* __restric
     for (int q = 0; q < CH; ++q) {
       if (q < cnt) {
 #pragma unroll
-        for (int c = 0; c < QC; ++c) {
-#pragma unroll
-          for (int k = 0; k < NR; ++k)
-            acc[k] = __builtin_fmaf(tv[q][c], Xs[q * NBS + cq * QC + c][k], acc[k]);
-        }
+        for (int c = 0; c < QC; ++c)
+          acc = __builtin_fmaf(tv[q][c], Xs[q * NBS + cq * QC + c], acc);
       }
     }
     __syncthreads();
   }
 
+  // the sum of the four column quarters' parts, in a fixed order
+  auto total = [&]() { return ((Red[0][row] + Red[1][row]) + Red[2][row]) + Red[3][row]; };
   // right-hand side of the diagonal block: B_i - sum_j T_ij X_j (over the
   // blocks summed so far)
-#pragma unroll
-  for (int k = 0; k < NR; ++k) Red[cq][row][k] = acc[k];
+  Red[cq][row] = acc;
   __syncthreads();
-  for (int k = cq; k < NR; k += 4) {
-    const float sum = ((Red[0][row][k] + Red[1][row][k]) + Red[2][row][k]) + Red[3][row][k];
-    const float bv = NR == 1 ? bpf : b[grc + (k < nrhs ? k : 0) * ldb];
-    Xs[row][k] = (gr < n && k < nrhs) ? bv - sum : 0.0f;
-  }
+  if (cq == 0) Xs[row] = gr < n ? bv - total() : 0.0f;
   __syncthreads();
   // X_i = (T_ii)^-1 (B_i - ...)  (with the fold: C)
-  float y[NR];
+  float y = 0.0f;
 #pragma unroll
-  for (int k = 0; k < NR; ++k) y[k] = 0.0f;
-#pragma unroll
-  for (int c = 0; c < QC; ++c) {
-    const float d = NR == 1 ? Ds[row][cq * QC + c] : dv[c];
-#pragma unroll
-    for (int k = 0; k < NR; ++k) y[k] = __builtin_fmaf(d, Xs[cq * QC + c][k], y[k]);
-  }
-#pragma unroll
-  for (int k = 0; k < NR; ++k) Red[cq][row][k] = y[k];
+  for (int c = 0; c < QC; ++c) y = __builtin_fmaf(Ds[row][cq * QC + c], Xs[cq * QC + c], y);
+  Red[cq][row] = y;
   __syncthreads();
-  if constexpr (FOLD) {
-    if (fold) {
-      // C (right-hand sides k = cq + 4 j in lane (row, cq)), then the near
-      // block: X_i = C - M X_near
-      constexpr int NJ = (NR + 3) / 4;
-      float cv[NJ];
+  float xv = cq == 0 ? total() : 0.0f;
+  if (fold) {
+    // then the near block: X_i = C - M X_near
+    __syncthreads();  // (Red and Xs are rewritten below)
+    stage_blocks(tk - 1, 1);
+    float z = 0.0f;
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        const int k = cq + 4 * j;
-        cv[j] = k < NR ? ((Red[0][row][k] + Red[1][row][k]) + Red[2][row][k]) + Red[3][row][k]
-                       : 0.0f;
-      }
-      __syncthreads();  // (Red and Xs are rewritten below)
-      stage_blocks(tk - 1, 1);
-      float z[NR];
-#pragma unroll
-      for (int k = 0; k < NR; ++k) z[k] = 0.0f;
-#pragma unroll
-      for (int c = 0; c < QC; ++c) {
-#pragma unroll
-        for (int k = 0; k < NR; ++k) z[k] = __builtin_fmaf(mv[c], Xs[cq * QC + c][k], z[k]);
-      }
-#pragma unroll
-      for (int k = 0; k < NR; ++k) Red[cq][row][k] = z[k];
-      __syncthreads();
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        const int k = cq + 4 * j;
-        if (k < NR && k < nrhs && gr < n) {
-          const float xv =
-              cv[j] - (((Red[0][row][k] + Red[1][row][k]) + Red[2][row][k]) + Red[3][row][k]);
-          b[gr + k * ldb] = xv;  // the caller's copy
-          __hip_atomic_store(&tags[gr + (int64_t)k * n],
-                             (1ull << 32) | (unsigned long long)__float_as_uint(xv),
-                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-      }
-    }
+    for (int c = 0; c < QC; ++c) z = __builtin_fmaf(mv[c], Xs[cq * QC + c], z);
+    Red[cq][row] = z;
+    __syncthreads();
+    if (cq == 0) xv -= total();
   }
-  for (int k = cq; k < NR && !fold; k += 4) {
-    const float xv = ((Red[0][row][k] + Red[1][row][k]) + Red[2][row][k]) + Red[3][row][k];
-    if (gr < n && k < nrhs) {
-      b[gr + k * ldb] = xv;  // the caller's copy
-      __hip_atomic_store(&tags[gr + (int64_t)k * n],
-                         (1ull << 32) | (unsigned long long)__float_as_uint(xv), __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-    }
+  if (cq == 0 && gr < n) {
+    b[gr] = xv;  // the caller's copy
+    __hip_atomic_store(&tags[gr], (1ull << 32) | (unsigned long long)__float_as_uint(xv),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
