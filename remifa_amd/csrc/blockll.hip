@@ -145,9 +145,8 @@ __device__ __forceinline__ unsigned pack_h2(float a, float b) {
 // The pivots of one 32-entry block of a unit, in order (see the header).
 // The tile's rows are read from LDS two pivots ahead of their use; the
 // owner of pivot k finds its scale in its own part of row k (entry k).
-template <int MODE>
 __device__ __forceinline__ void solve_block(float (&x)[16], const float (*m)[32], int lh) {
-  using Sm = Sem<MODE>;
+  using Sm = BlockSem;
   constexpr int PF = 3;  // row buffers in flight
   float4 mv[PF][4];
   auto fetch = [&](int k) {
@@ -189,11 +188,11 @@ __device__ __forceinline__ void solve_block(float (&x)[16], const float (*m)[32]
 // the slice at column so, on one wavefront. T = the role's table and pan
 // the other factor's op-rounded vectors of the tile ([e][k], k < so), both
 // in LDS.
-template <int MODE, int KC>
+template <int KC>
 __device__ __forceinline__ void do_unit(const BlkArgs& g, const RoleTab& T,
                                         const _Float16 (*pan)[PP], int role, int64_t v0,
                                         int so) {
-  using Sm = Sem<MODE>;
+  using Sm = BlockSem;
   const int lane = threadIdx.x & 63, l32 = lane & 31, lh = lane >> 5;
   const int64_t v = v0 + l32;
   const bool ok = v < g.updm;
@@ -250,7 +249,7 @@ __device__ __forceinline__ void do_unit(const BlkArgs& g, const RoleTab& T,
   // block 0
 #pragma unroll
   for (int r = 0; r < 16; ++r) x0[r] = -acc0[r];
-  solve_block<MODE>(x0, T.m[0], lh);
+  solve_block(x0, T.m[0], lh);
   // block 1: its part of the sum over block 0 joins the same accumulator
   // (B operand: op(x0) rearranged across the halves, see the header)
 #pragma unroll
@@ -267,7 +266,7 @@ __device__ __forceinline__ void do_unit(const BlkArgs& g, const RoleTab& T,
   }
 #pragma unroll
   for (int r = 0; r < 16; ++r) x1[r] = -acc1[r];
-  solve_block<MODE>(x1, T.m[1], lh);
+  solve_block(x1, T.m[1], lh);
   if (!ok) return;
   // the factors (fp16) and the op-rounded copy for later slices
   half_t* oc = (role ? g.uop : g.lop) + vc * ldo + so + 4 * lh;
@@ -302,9 +301,9 @@ __device__ __forceinline__ void do_unit(const BlkArgs& g, const RoleTab& T,
 
 // solve_block for N units of one role at once (the same table rows feed
 // all of them; their pivot chains interleave)
-template <int MODE, int N>
+template <int N>
 __device__ __forceinline__ void solve_blocks(float (&x)[N][16], const float (*m)[32], int lh) {
-  using Sm = Sem<MODE>;
+  using Sm = BlockSem;
   constexpr int PF = 3;  // row buffers in flight
   float4 mv[PF][4];
   auto fetch = [&](int k) {
@@ -350,7 +349,7 @@ __device__ __forceinline__ void solve_blocks(float (&x)[N][16], const float (*m)
 // do_unit for N units of one role at once (vectors from v0[n]): the same
 // arithmetic per unit; the other factor's tile vectors and the table rows
 // are read once for all of them and their chains interleave.
-template <int MODE, int KC, int N>
+template <int KC, int N>
 __device__ __forceinline__ void do_units(const BlkArgs& g, const RoleTab& T,
                                          const _Float16 (*pan)[PP], int role,
                                          const int64_t (&v0)[N], int so) {
@@ -422,7 +421,7 @@ __device__ __forceinline__ void do_units(const BlkArgs& g, const RoleTab& T,
   for (int n = 0; n < N; ++n)
 #pragma unroll
     for (int r = 0; r < 16; ++r) x0[n][r] = -acc0[n][r];
-  solve_blocks<MODE, N>(x0, T.m[0], lh);
+  solve_blocks<N>(x0, T.m[0], lh);
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks) {
     const int g0 = 8 * ks, g1 = 8 * ks + 4;
@@ -443,7 +442,7 @@ __device__ __forceinline__ void do_units(const BlkArgs& g, const RoleTab& T,
   for (int n = 0; n < N; ++n)
 #pragma unroll
     for (int r = 0; r < 16; ++r) x1[n][r] = -acc1[n][r];
-  solve_blocks<MODE, N>(x1, T.m[1], lh);
+  solve_blocks<N>(x1, T.m[1], lh);
 #pragma unroll
   for (int n = 0; n < N; ++n) {
     if (!ok[n]) continue;
@@ -522,9 +521,9 @@ __device__ __forceinline__ void stage_panels(_Float16 (*pan0)[PP], const half_t*
   }
 }
 
-template <int MODE, bool PUB>
+template <bool PUB>
 __device__ void diagonal_role(const BlkArgs& g, DiagLds& S) {
-  using Sm = Sem<MODE>;
+  using Sm = BlockSem;
   const int t = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(t / 64);
   const int i = t & 63, l32 = i & 31, lh = i >> 5;
@@ -572,7 +571,7 @@ __device__ void diagonal_role(const BlkArgs& g, DiagLds& S) {
     for (int jj = 0; jj < TP; ++jj) x[jj] = S.f.tt[i][cb + jj];
     __syncthreads();
     // 2. the factorization (ib = 32)
-    tile_factor<MODE, 32>(S.f.fac, x, 32, w, i);
+    tile_factor<32>(S.f.fac, x, w, i);
     __syncthreads();
     const float rk = S.f.fac.R[i];
     // 3. the factored tile: fp16 factors, the slice table (LDS, then copied
@@ -652,20 +651,19 @@ __device__ void diagonal_role(const BlkArgs& g, DiagLds& S) {
           __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         }
       }
-      do_unit<MODE, 14>(g, S.tab.role[role], S.pan[role], role, so + SW + NV * u, so);
+      do_unit<14>(g, S.tab.role[role], S.pan[role], role, so + SW + NV * u, so);
     }
     __syncthreads();
   }
 }
 
-template <int MODE>
 __global__ void __launch_bounds__(BLT) blockll_diag_kernel(BlkArgs g) {
   __shared__ DiagLds S;
-  diagonal_role<MODE, false>(g, S);
+  diagonal_role<false>(g, S);
 }
 
 // far workgroups 0 .. nfw-1 take rows of L, the others columns of U
-template <int MODE, int KC>
+template <int KC>
 __device__ __forceinline__ void far_body(const BlkArgs& g) {
   __shared__ _Float16 pan[SW][PP];
   __shared__ RoleTab tab;
@@ -684,16 +682,16 @@ __device__ __forceinline__ void far_body(const BlkArgs& g) {
     stage_panel(pan, role ? g.lop : g.uop, g.ldo, so);
     __syncthreads();
     for (int u = fr * (BLT / 64) + w; u < g.nfu; u += g.nfw * (BLT / 64))
-      do_unit<MODE, KC>(g, tab, pan, role, g.nb + (int64_t)NV * u, so);
+      do_unit<KC>(g, tab, pan, role, g.nb + (int64_t)NV * u, so);
     __syncthreads();
   }
 }
 // (at most 128 registers: two far workgroups, or one beside an update GEMM
 // workgroup, fit on a CU)
-template <int MODE, int KC>
+template <int KC>
 __global__ void __launch_bounds__(BLT) __attribute__((amdgpu_waves_per_eu(4)))
 blockll_far_kernel(BlkArgs g) {
-  far_body<MODE, KC>(g);
+  far_body<KC>(g);
 }
 
 // One-launch form, far role: helper hx of nhelp; its wavefronts take units
@@ -703,7 +701,6 @@ blockll_far_kernel(BlkArgs g) {
 // while it is below the next tile, slices s <= b/2 - 2, its progress
 // published after each), then the far units (role f % 2, unit f / 2 for
 // f = q - 2 ndu).
-template <int MODE>
 __device__ void helper_role(const BlkArgs& g, DiagLds& S, int hx, int nhelp) {
   const int t = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(t / 64);
@@ -745,7 +742,7 @@ __device__ void helper_role(const BlkArgs& g, DiagLds& S, int hx, int nhelp) {
     for (; q < tot && q < 2 * ndu; q += hw) {
       const int role = q & 1, b = 4 + (q >> 1);
       if (2 * s + 4 > b) continue;  // the diagonal role's from here on
-      do_unit<MODE, 8>(g, S.tab.role[role], S.pan[role], role, (int64_t)NV * b, so);
+      do_unit<8>(g, S.tab.role[role], S.pan[role], role, (int64_t)NV * b, so);
       // (this wavefront's stores have reached the L2; the release store
       // writes it back)
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -760,13 +757,13 @@ __device__ void helper_role(const BlkArgs& g, DiagLds& S, int hx, int nhelp) {
       if (q + 2 * hw < tot) {
         const int64_t v0[3] = {g.nb + (int64_t)NV * (f >> 1), g.nb + (int64_t)NV * ((f + hw) >> 1),
                                g.nb + (int64_t)NV * ((f + 2 * hw) >> 1)};
-        do_units<MODE, 4, 3>(g, S.tab.role[role], S.pan[role], role, v0, so);
+        do_units<4, 3>(g, S.tab.role[role], S.pan[role], role, v0, so);
         q += hw;
       } else if (q + hw < tot) {
         const int64_t v0[2] = {g.nb + (int64_t)NV * (f >> 1), g.nb + (int64_t)NV * ((f + hw) >> 1)};
-        do_units<MODE, 4, 2>(g, S.tab.role[role], S.pan[role], role, v0, so);
+        do_units<4, 2>(g, S.tab.role[role], S.pan[role], role, v0, so);
       } else {
-        do_unit<MODE, 8>(g, S.tab.role[role], S.pan[role], role, g.nb + (int64_t)NV * (f >> 1),
+        do_unit<8>(g, S.tab.role[role], S.pan[role], role, g.nb + (int64_t)NV * (f >> 1),
                          so);
       }
     }
@@ -774,7 +771,6 @@ __device__ void helper_role(const BlkArgs& g, DiagLds& S, int hx, int nhelp) {
   }
 }
 
-template <int MODE>
 __global__ void __launch_bounds__(BLT) blockll_fused_kernel(BlkArgs g, int nhelp) {
   __shared__ DiagLds S;
   __shared__ int s_tk;
@@ -783,9 +779,9 @@ __global__ void __launch_bounds__(BLT) blockll_fused_kernel(BlkArgs g, int nhelp
   __syncthreads();
   const int tk = s_tk;
   if (tk == 0)
-    diagonal_role<MODE, true>(g, S);
+    diagonal_role<true>(g, S);
   else if (tk > 0 && tk <= nhelp)  // (any other ticket: counter not reset; the waits report it)
-    helper_role<MODE>(g, S, tk - 1, nhelp);
+    helper_role(g, S, tk - 1, nhelp);
 }
 
 __global__ void blockll_sync_reset_kernel(int* sync) {
@@ -875,7 +871,7 @@ int blockll_launch(remifa_handle_t h, void* base, int64_t m, int64_t nb, int64_t
     g.tbase = seq[1];
     seq[1] += 1 + nhelp;
     timer_begin(h, KC_PANEL, bytes, 4);
-    blockll_fused_kernel<SM_F32_TC><<<1 + nhelp, BLT, 0, h->stream>>>(g, nhelp);
+    blockll_fused_kernel<<<1 + nhelp, BLT, 0, h->stream>>>(g, nhelp);
     RF_HIP(hipGetLastError());
     timer_end(h);
     return 0;
@@ -883,12 +879,12 @@ int blockll_launch(remifa_handle_t h, void* base, int64_t m, int64_t nb, int64_t
   g.tbase = 0;
   g.epoch = 0;
   timer_begin(h, KC_PANEL, bytes, 2);
-  blockll_diag_kernel<SM_F32_TC><<<1, BLT, 0, h->stream>>>(g);
+  blockll_diag_kernel<<<1, BLT, 0, h->stream>>>(g);
   RF_HIP(hipGetLastError());
   timer_end(h);
   if (g.nfu > 0) {
     timer_begin(h, KC_PANEL, bytes, 3);
-    blockll_far_kernel<SM_F32_TC, 8><<<2 * g.nfw, BLT, 0, h->stream>>>(g);
+    blockll_far_kernel<8><<<2 * g.nfw, BLT, 0, h->stream>>>(g);
     RF_HIP(hipGetLastError());
     timer_end(h);
   }

@@ -21,64 +21,47 @@ enum SubMode {
 };
 
 __device__ __forceinline__ float r16(float x) { return (float)(half_t)x; }
-__device__ __forceinline__ float rbf(float x) { return bf16_bits_to_f32(f32_to_bf16_bits(x)); }
 
+// c - acc, a cross-block sum's subtraction, rounded to the panel precision
 template <int MODE>
 struct Sem {
-  static constexpr bool HALF = MODE >= SM_F16_TC;  // fp16 storage and panel arithmetic
-  // operand rounding of the cross-block updates
-  static __device__ __forceinline__ float op(float x) {
-    if constexpr (MODE == SM_F32_TC) return r16(x);
-    if constexpr (MODE == SM_F16_BF) return rbf(x);
-    return x;  // fp32, or already fp16-valued
-  }
-  // panel arithmetic
-  static __device__ __forceinline__ float rcp(float x) {
-    float r = 1.0f / x;
-    return HALF ? r16(r) : r;
-  }
-  static __device__ __forceinline__ float mul(float a, float b) {
-    float r = a * b;  // exact for fp16 inputs
-    return HALF ? r16(r) : r;
-  }
-  static __device__ __forceinline__ float fnma(float a, float b, float c) {
-    if constexpr (HALF)
-      return (float)__builtin_fmaf16(-(half_t)a, (half_t)b, (half_t)c);
-    else
-      return __builtin_fmaf(-a, b, c);
-  }
-  // cross-block product sums: operands are already op-rounded
-  static __device__ __forceinline__ float acc_add(float acc, float a, float b) {
-    if constexpr (MODE == SM_F16_H)
-      return (float)__builtin_fmaf16((half_t)a, (half_t)b, (half_t)acc);
-    else
-      return __builtin_fmaf(a, b, acc);
-  }
-  // c - acc, rounded to the panel precision
   static __device__ __forceinline__ float apply(float c, float acc) {
     if constexpr (MODE == SM_F16_H) return (float)((half_t)c - (half_t)acc);
-    float r = c - acc;
-    return HALF ? r16(r) : r;
+    const float r = c - acc;
+    return MODE >= SM_F16_TC ? r16(r) : r;
   }
+};
+
+// the block kernel's arithmetic: fp32 data, cross-block sums of fp16 operands
+struct BlockSem {
+  static __device__ __forceinline__ float op(float x) { return r16(x); }
+  static __device__ __forceinline__ float rcp(float x) { return 1.0f / x; }
+  static __device__ __forceinline__ float mul(float a, float b) { return a * b; }
+  static __device__ __forceinline__ float fnma(float a, float b, float c) {
+    return __builtin_fmaf(-a, b, c);
+  }
+  static __device__ __forceinline__ float acc_add(float acc, float a, float b) {
+    return __builtin_fmaf(a, b, acc);
+  }
+  static __device__ __forceinline__ float apply(float c, float acc) { return c - acc; }
 };
 
 // ---------------------------------------------------------------------------
 // 1. the diagonal tile, blocked by 8-column panels: eight wavefronts, lane i
 // holds row i, wavefront w owns columns 8w..8w+7 in registers. Stage g:
 // wavefront g factors its panel (8 pivots, the pivot row broadcast with
-// readlane inside the wavefront) and shares the multipliers through LDS; after one barrier every
-// wavefront right of it applies the panel's 8 pivots to its own columns in
-// pivot order. Every entry receives the same sequence of fused updates as in
-// a pivot-by-pivot elimination. ib (a multiple of 8) decides where the block
-// boundaries fall: at a block boundary the block sums run as runtime loops
-// over LDS copies of the operands.
+// readlane inside the wavefront) and shares the multipliers through LDS; after
+// one barrier every wavefront right of it applies the panel's 8 pivots to its
+// own columns in pivot order. Every entry receives the same sequence of fused
+// updates as in a pivot-by-pivot elimination. At the boundary of the blocks of
+// IB = SW - KM columns the block sums run over LDS copies of the operands.
 constexpr int TP = 8;  // panel width = columns per wavefront
 
 // Row pitches are 16-byte multiples so that a lane publishes its 8 values
 // with two 16-byte stores; 48-, 144- and 272-byte pitches keep 16
 // consecutive lanes on distinct banks. The op-rounded copies feed only the
-// block sums, which read columns / rows below the last block's start: KM =
-// SW - ib of them are kept.
+// block sums, which read columns / rows below the last block's start: KM of
+// them are kept.
 template <int KM>
 struct __attribute__((aligned(16))) TileLdsT {
   __attribute__((aligned(16))) float Lp[2][SW][TP + 4];  // multipliers of the current panel
@@ -100,16 +83,16 @@ __device__ __forceinline__ float bcast_lane(float v, int lane) {
 // The tile factorization proper, on eight wavefronts: lane i of wavefront w
 // holds x[jj] = T[i][8 w + jj]; on return the same registers hold the
 // factors (multipliers below the diagonal, U on and above it) and S.R the
-// reciprocals of the pivots. ib is the block size (8, 16, 32 or 64, with
-// SW - ib <= KM).
-template <int MODE, int KM>
-__device__ __forceinline__ void tile_factor(TileLdsT<KM>& S, float (&x)[TP], int ib, int w, int i) {
-  using Sm = Sem<MODE>;
+// reciprocals of the pivots.
+template <int KM>
+__device__ __forceinline__ void tile_factor(TileLdsT<KM>& S, float (&x)[TP], int w, int i) {
+  using Sm = BlockSem;
+  constexpr int IB = SW - KM;
   const int cb = w * TP;
   for (int g = 0; g < SW / TP; ++g) {
     const int p0 = g * TP;         // first pivot of the panel
-    const int kb = p0 - p0 % ib;   // ib block holding it: [kb, kend)
-    const int kend = kb + ib;
+    const int kb = p0 - p0 % IB;   // block holding it: [kb, kend)
+    const int kend = kb + IB;
     // (every wavefront takes every stage: the barrier below needs all eight;
     // columns left of the panel are final and take no work)
     if (p0 == kb && kb > 0 && w >= g) {
