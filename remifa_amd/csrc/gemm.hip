@@ -386,6 +386,10 @@ int launch_mfma(remifa_handle_t h, GemmArgs g, int split, bool vec) {
   constexpr bool PRE = false;
   if (vec)
     gemm_mfma_kernel<OPK, OutT, BM, BN, WM, WN, BK, true, PRE><<<grid, 256, 0, h->stream>>>(g);
+  else if (BM == 32 && g.lda < OpTraits<OPK>::CH)
+    // (a few contiguous rows: no chunk of a column can be read whole)
+    gemm_mfma_kernel<OPK, OutT, BM, BN, WM, WN, BK, false, PRE, BM == 32>
+        <<<grid, 256, 0, h->stream>>>(g);
   else
     gemm_mfma_kernel<OPK, OutT, BM, BN, WM, WN, BK, false, PRE><<<grid, 256, 0, h->stream>>>(g);
   RF_HIP(hipGetLastError());

@@ -159,7 +159,8 @@ struct TileLdsGeom {
 
 // One workgroup's tile: `bid` is its tile index (remapped below), `bz` its
 // K slice; As0 / Bs0: two LDS buffers each of A and B slabs.
-template <int OPK, typename OutT, int BM, int BN, int WM, int WN, int BK, bool VEC, bool PRELOAD>
+template <int OPK, typename OutT, int BM, int BN, int WM, int WN, int BK, bool VEC, bool PRELOAD,
+          bool MASKED = false>
 __device__ __forceinline__ void gemm_mfma_body(const GemmArgs& g, int bid, int bz, bool split,
                                                typename OpTraits<OPK>::Lds* As0,
                                                typename OpTraits<OPK>::Lds* Bs0) {
@@ -426,34 +427,33 @@ __device__ __forceinline__ void gemm_mfma_body(const GemmArgs& g, int bid, int b
       run(std::integral_constant<bool, true>{});
     else
       run(std::integral_constant<bool, false>{});
+  } else if constexpr (MASKED) {
+    run(std::integral_constant<bool, false>{});  // every slab element by element
   } else {
     // A chunk past the last row reads on into the next column, except in A's
     // last column; a short slab's chunks would leave the K range: that slab is
-    // masked (lda >= CH keeps the last column but one inside A). No other slab:
-    // the masked loop alone.
+    // masked (lda >= CH keeps the last column but one inside A)
     const bool mask_last =
         klen % BK != 0 || (kend == g.K && g.M % CH != 0 && m0 + BM >= g.M);
     const int nfull = !(off32 && g.lda >= CH) ? 0 : (mask_last ? nk - 1 : nk);
-    if (nfull <= 0) {
-      run(std::integral_constant<bool, false>{});
-    } else {
-      auto load = [&](int kt) {
-        if (kt < nfull)
-          load_slab(kt, std::integral_constant<bool, true>{});
-        else
-          load_slab(kt, std::integral_constant<bool, false>{});
-      };
+    auto load = [&](int kt) {
+      if (kt < nfull)
+        load_slab(kt, std::integral_constant<bool, true>{});
+      else
+        load_slab(kt, std::integral_constant<bool, false>{});
+    };
+    if (nk > 0) {
       load(0);
       store_tiles(0, std::integral_constant<bool, true>{});
+    }
+    __syncthreads();
+    for (int kt = 0; kt < nk; ++kt) {
+      const int buf = kt & 1;
+      const bool more = kt + 1 < nk;
+      if (more) load(kt + 1);
+      compute(buf);
+      if (more) store_tiles(buf ^ 1, std::integral_constant<bool, true>{});
       __syncthreads();
-      for (int kt = 0; kt < nk; ++kt) {
-        const int buf = kt & 1;
-        const bool more = kt + 1 < nk;
-        if (more) load(kt + 1);
-        compute(buf);
-        if (more) store_tiles(buf ^ 1, std::integral_constant<bool, true>{});
-        __syncthreads();
-      }
     }
   }
 
@@ -492,14 +492,15 @@ __device__ __forceinline__ void gemm_mfma_body(const GemmArgs& g, int bid, int b
   }
 }
 
-template <int OPK, typename OutT, int BM, int BN, int WM, int WN, int BK, bool VEC, bool PRELOAD>
+template <int OPK, typename OutT, int BM, int BN, int WM, int WN, int BK, bool VEC, bool PRELOAD,
+          bool MASKED = false>
 __global__ void __launch_bounds__(256) gemm_mfma_kernel(GemmArgs g) {
   using L = typename OpTraits<OPK>::Lds;
   using GEO = TileLdsGeom<OPK, BM, BN, BK>;
   __shared__ __attribute__((aligned(16))) L As[2 * GEO::A_ELEMS];
   __shared__ __attribute__((aligned(16))) L Bs[2 * GEO::B_ELEMS];
-  gemm_mfma_body<OPK, OutT, BM, BN, WM, WN, BK, VEC, PRELOAD>(g, blockIdx.x, blockIdx.z,
-                                                              gridDim.z > 1, As, Bs);
+  gemm_mfma_body<OPK, OutT, BM, BN, WM, WN, BK, VEC, PRELOAD, MASKED>(
+      g, blockIdx.x, blockIdx.z, gridDim.z > 1, As, Bs);
 }
 
 // Two independent GEMMs in one launch (no split-K): workgroups [0, nt0) run
