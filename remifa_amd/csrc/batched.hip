@@ -4,9 +4,10 @@
 //
 // One persistent launch: a grid of as many workgroups as the chip holds (or
 // as there are matrices) takes matrices from an atomic queue (callers order
-// the batch largest first, so the queue is a longest-processing-time schedule). A workgroup factors its
-// matrix right-looking with 32-wide panels, which is the reference's RL
-// driver with nb = ib = 32 (src/lu_nopiv.hxx:53-208): per panel
+// the batch largest first, so the queue is a longest-processing-time
+// schedule). A workgroup factors its matrix right-looking with 32-wide
+// panels, which is the reference's RL driver with nb = ib = 32
+// (src/lu_nopiv.hxx:53-208): per panel
 //  1. the 32 pivots of the panel: lane i keeps row i of the panel in
 //     registers; wavefront 0 factors the top 32 x 32 block (pivot rows by
 //     readlane), then every lane takes its row below against U11 from LDS,
@@ -310,7 +311,8 @@ __global__ void __launch_bounds__(BT) batched_getrs_kernel(int count, const int*
   // row i (in bounds) of the columns k0 .. k0 + kw - 1, the last repeated
   auto read_row = [&](int i, int k0, int kw, float (&w)[32]) {
 #pragma unroll
-    for (int k = 0; k < 32; ++k) w[k] = (a + (int64_t)(k0 + (k < kw ? k : kw - 1)) * ld)[(unsigned)i];
+    for (int k = 0; k < 32; ++k)
+      w[k] = (a + (int64_t)(k0 + (k < kw ? k : kw - 1)) * ld)[(unsigned)i];
   };
   // x_i -= the row's products with x_k0 .. in order
   auto update = [&](int i, int k0, int kw, const float (&w)[32]) {

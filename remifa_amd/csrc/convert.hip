@@ -1,6 +1,7 @@
-// Precision conversion of column-major blocks (src/convert.cu:324-360). HBM-bound streaming kernels: each thread takes 8
-// consecutive rows of 4 columns with vector accesses, so a wavefront reads 512
-// consecutive elements of a column; the y grid dimension walks the columns.
+// Precision conversion of column-major blocks (src/convert.cu:324-360).
+// HBM-bound streaming kernels: each thread takes 8 consecutive rows of 4
+// columns with vector accesses, so a wavefront reads 512 consecutive elements
+// of a column; the y grid dimension walks the columns.
 #include "common.hpp"
 
 namespace remifa {

@@ -711,7 +711,8 @@ int gemm_pair_launch(remifa_handle_t h, int ctype, int in_t, int out_t, int64_t 
   const bool v0 = vec_ok(a0, lda0, b0, ldb0, m0), v1 = vec_ok(a1, lda1, b1, ldb1, m1);
   const bool pair = opk >= 0 && k > 0 && m0 > 0 && n0 > 0 && m1 > 0 && n1 > 0 && t0 == T256x32 &&
                     t1 == T32x256 && s0 <= 1 && s1 <= 1 && h->split_k <= 0 && h->gemm_tile < 0 &&
-                    v0 == v1 && (out_t == REMIFA_R_32F || (out_t == REMIFA_R_16F && opk != OPK_F32));
+                    v0 == v1 &&
+                    (out_t == REMIFA_R_32F || (out_t == REMIFA_R_16F && opk != OPK_F32));
   if (!pair) {
     RF_CHECK(gemm_launch(h, ctype, in_t, out_t, m0, n0, k, -1.0f, a0, lda0, b0, ldb0, 1.0f, c0,
                          ldc0));
